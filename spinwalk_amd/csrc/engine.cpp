@@ -95,6 +95,7 @@ struct sw_sequence {
     bool exc_valid = false;
     float key_lin = 0, key_quad = 0; int32_t key_ndummy = -1;
     float RF_FA0 = 0, RF_PH0 = 0;
+    bool closed = false;             // no crossing probability between two tissues is above 0
     // The tables that shape a walk's trajectory and relaxation, byte for byte:
     // diffusivity, P_XY, T1/T2 and every event time.  Tiles whose sequences have
     // equal signatures (and equal draws, geometry and start positions) walk the
@@ -659,6 +660,10 @@ SW_API int sw_sequence_create(sw_engine *e, const sw_params *p, const sw_seq *q,
         T1d[i] = (double)q->T1_ms[i] * 1e-3;
         T2d[i] = (double)q->T2_ms[i] * 1e-3;
     }
+    sq->closed = true;
+    for (uint32_t i = 0; i < ns; i++)
+        for (uint32_t j = 0; j < ns; j++)
+            if (i != j && !(q->pXY[i * ns + j] <= 0.f)) sq->closed = false;
     std::vector<sw::RfPulse> rf(q->n_rf);
     for (uint32_t k = 0; k < q->n_rf; k++) {
         const float fa = q->RF_FA_deg[k], phs = q->RF_PH_deg[k];
@@ -836,6 +841,7 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
     a.g2d = (float)(1e-3 * p->timestep_us * 1e-6 * kGamma * kRad2Deg);
     a.diffusivity = q->diffusivity; a.pXY = q->pXY; a.T1s = q->T1s; a.T2s = q->T2s; a.T1d = q->T1d; a.T2d = q->T2d;
     a.n_sub = q->n_sub;
+    a.closed = q->closed ? 1u : 0u;
     // The tissue tables go to LDS beside the per-axis tables of the 32-bit mode
     // when both fit its 64 KiB (a walk in the 64-bit mode ignores the flag).
     a.tissue_lds = (o->rng != SW_RNG_REPLAY && q->n_sub <= sw::kTissueLdsMax &&
@@ -995,7 +1001,7 @@ struct sw_batch {
     sw::Excitation *d_exc = nullptr;             // every tile's excitation table
     uint32_t *d_order = nullptr;                 // every tile's visiting order
     double *d_partial = nullptr;                 // echo-reduction scratch
-    struct Group { bool cross; int views; uint32_t offset, n_slots; };
+    struct Group { int variant; int views; uint32_t offset, n_slots; };
     std::vector<Group> groups;
     struct Reduce { const void *M1; int f64; const uint8_t *T; uint32_t n, n_te, n_sub; double *out; };
     std::vector<Reduce> reduces;
@@ -1004,9 +1010,9 @@ struct sw_batch {
     bool mixed = false;                          // 64-bit mode over items in both packed layouts
     size_t lds = 0;                              // LDS of a workgroup: per-axis tables, then tissue tables (32-bit mode)
     // what the chunk table is built from: per walk unit (a single tile, or a
-    // fused group of tiles), its CROSS_FOV group, spins, steps per spin, phantom
-    // records, views (1: d_items[index]; kMaxViews: d_fused[index])
-    struct Tile { bool cross; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; };
+    // fused group of tiles), its kernel variant (launch_walk_batch), spins, steps
+    // per spin, phantom records, views (1: d_items[index]; kMaxViews: d_fused[index])
+    struct Tile { int variant; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; };
     std::vector<Tile> tiles;
     uint32_t n_fused_tiles = 0;                  // tiles walked inside fused units
     sw_batch_schedule sched{};
@@ -1051,7 +1057,7 @@ hipError_t batch_enqueue(const sw_batch *b, hipStream_t s) {
     for (const auto &g : b->groups) {
         const void *items = g.views == 1 ? (const void *)b->d_items : (const void *)b->d_fused;
         err = sw::launch_walk_batch(items, b->d_chunks + g.offset, g.n_slots, b->sched.chunk_spins,
-                                    b->sched.spins_per_lane, g.views, b->rng, b->field, b->prec, g.cross,
+                                    b->sched.spins_per_lane, g.views, b->rng, b->field, b->prec, g.variant,
                                     b->idx32 ? sw::ADDR_32 : b->mixed ? sw::ADDR_64_MIXED : sw::ADDR_64,
                                     lds, s);
         if (err != hipSuccess) return err;
@@ -1075,7 +1081,7 @@ hipError_t batch_enqueue(const sw_batch *b, hipStream_t s) {
 // and 1 for Kahan + int16 (66.5 against 68.3).  sw_batch_tune searches around it.
 constexpr sw_batch_schedule kDefaultSchedule = {256u, 1u << 20, 4u, 1u, 0u, 8u};
 
-// The chunk table of a schedule: per CROSS_FOV group and walk kind (single or
+// The chunk table of a schedule: per kernel variant and walk kind (single or
 // fused), each walk unit's chunks of sc.chunk_spins spins split into 8
 // contiguous parts (one per XCD; a part is one spatial region of the unit,
 // since chunks follow the visiting order).  Within
@@ -1092,11 +1098,11 @@ void build_chunk_table(const sw_batch &b, const sw_batch_schedule &sc, std::vect
     groups.clear();
     *kinds = 0;
     const uint32_t cs = sc.chunk_spins * sc.spins_per_lane;
-    for (int grp = 0; grp < 4; grp++) {
-        const int cross = grp & 1, views = grp < 2 ? 1 : sw::kMaxViews;
+    for (int grp = 0; grp < 2 * sw::VARIANTS; grp++) {
+        const int variant = grp % sw::VARIANTS, views = grp < sw::VARIANTS ? 1 : sw::kMaxViews;
         std::vector<uint32_t> idx;
         for (uint32_t i = 0; i < (uint32_t)b.tiles.size(); i++)
-            if (b.tiles[i].cross == (cross != 0) && b.tiles[i].views == views && b.tiles[i].n_local) idx.push_back(i);
+            if (b.tiles[i].variant == variant && b.tiles[i].views == views && b.tiles[i].n_local) idx.push_back(i);
         if (idx.empty()) continue;
         auto cost = [&](uint32_t i) { return b.tiles[i].cost; };
         std::stable_sort(idx.begin(), idx.end(), [&](uint32_t x, uint32_t y) { return cost(x) > cost(y); });
@@ -1143,7 +1149,7 @@ void build_chunk_table(const sw_batch &b, const sw_batch_schedule &sc, std::vect
             per = std::max(per, lists[k].size());
         }
         sw_batch::Group g;
-        g.cross = cross != 0;
+        g.variant = variant;
         g.views = views;
         g.offset = (uint32_t)table.size();
         g.n_slots = (uint32_t)(8 * per);
@@ -1369,8 +1375,9 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
                 }
         const sw::WalkArgs &a0 = args[i];
         const uint64_t cost = (uint64_t)(a0.n_dummy + 1) * a0.n_timepoints;
+        const int variant = sw::walk_variant(a0, b->rng == SW_RNG_REPLAY);
         if (group.size() == 1) {
-            b->tiles.push_back({a0.cross_fov != 0, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size()});
+            b->tiles.push_back({variant, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size()});
             singles.push_back(a0);
             continue;
         }
@@ -1388,7 +1395,7 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
             w.M1 = x.M1; w.XYZ1 = x.XYZ1; w.T = x.T;
             w.counters = real ? x.counters : nullptr;      // a repeat of view 0 counts nothing
         }
-        b->tiles.push_back({a0.cross_fov != 0, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size()});
+        b->tiles.push_back({variant, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size()});
         fused.push_back(f);
         b->n_fused_tiles += (uint32_t)group.size();
     }

@@ -98,6 +98,52 @@ SW_HD U32x4 philox4x32_10_pre(uint32_t c0, uint32_t c1, uint32_t m_hi, uint32_t 
     return o;
 }
 
+// philox4x32_10_pre for a counter (att, spin, 0) whose attempt word `att` and key
+// are uniform across the wave: round 1's first product and round 2's second are
+// then scalar, and the words they meet fold on the scalar unit.
+SW_HD U32x4 philox4x32_10_uniform(uint64_t att, uint32_t m_hi, uint32_t m_lo, uint32_t k0, uint32_t k1) {
+    constexpr uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
+#if defined(__HIP_DEVICE_COMPILE__) && 0
+    asm volatile("" : "+s"(k0), "+s"(k1));
+#endif
+    uint32_t c0, c1, c2, c3;
+    {
+        const uint64_t p0 = (uint64_t)kPhiloxM0 * (uint32_t)att;          // round 1
+        const uint32_t s2 = (uint32_t)(p0 >> 32) ^ k1;
+        uint32_t s0 = (uint32_t)(att >> 32) ^ k0;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(s0));                                      // else it joins the vector words
+#endif
+        c0 = m_hi ^ s0;
+        k0 += W0; k1 += W1;
+        const uint64_t p1 = (uint64_t)kPhiloxM1 * s2;                     // round 2
+        const uint64_t q0 = (uint64_t)kPhiloxM0 * c0;
+        c0 = m_lo ^ ((uint32_t)(p1 >> 32) ^ k0);
+        c2 = (uint32_t)(q0 >> 32) ^ ((uint32_t)p0 ^ k1);
+        c3 = (uint32_t)q0;
+        k0 += W0; k1 += W1;
+        const uint64_t r0 = (uint64_t)kPhiloxM0 * c0, r1 = (uint64_t)kPhiloxM1 * c2;   // round 3
+        c0 = (uint32_t)(r1 >> 32) ^ ((uint32_t)p1 ^ k0);
+        c2 = xor3((uint32_t)(r0 >> 32), c3, k1);
+        c1 = (uint32_t)r1; c3 = (uint32_t)r0;
+        k0 += W0; k1 += W1;
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+    for (int r = 3; r < 10; ++r) {
+        const uint64_t p0 = (uint64_t)kPhiloxM0 * c0;
+        const uint64_t p1 = (uint64_t)kPhiloxM1 * c2;
+        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+        const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
+        c0 = n0; c1 = (uint32_t)p1; c2 = n2; c3 = (uint32_t)p0;
+        k0 += W0; k1 += W1;
+    }
+    U32x4 o;
+    o.v[0] = c0; o.v[1] = c1; o.v[2] = c2; o.v[3] = c3;
+    return o;
+}
+
 // 23-bit uniforms from the top bits of a word, built as floats in [1, 2).
 SW_HD float bits_to_float(uint32_t b) {
 #if defined(__HIP_DEVICE_COMPILE__)

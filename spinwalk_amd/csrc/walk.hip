@@ -1,14 +1,21 @@
 // walk.hip -- entry points of the walk kernels: dispatch to the kernel families
-// (walk_replay.hip, walk_philox.hip, walk_batch_philox.hip), the index mode of a
+// (walk_*.hip, one per family of walk_launch.hpp), the index mode of a
 // phantom, the counter fill kernel and the materialised production draws.
 #include "walk_impl.hpp"
 
 namespace sw {
 
 hipError_t launch_walk(const WalkArgs &a, int rng, int field, int prec, hipStream_t s) {
-    if (rng == 1) return launch_walk_replay(a, field, prec, s);
-    if (rng == 0) return launch_walk_philox(a, field, prec, s);
-    return hipErrorInvalidValue;
+    const bool half = field >= 2;
+    if (rng < 0 || rng > 1 || (prec == 2 && half)) return hipErrorInvalidValue;
+    switch (prec) {
+    case 0: return rng ? (half ? launch_walk_replay_f32_half : launch_walk_replay_f32_wide)(a, field, s)
+                       : (half ? launch_walk_philox_f32_half : launch_walk_philox_f32_wide)(a, field, s);
+    case 1: return rng ? (half ? launch_walk_replay_kahan_half : launch_walk_replay_kahan_wide)(a, field, s)
+                       : (half ? launch_walk_philox_kahan_half : launch_walk_philox_kahan_wide)(a, field, s);
+    case 2: return (rng ? launch_walk_replay_f64_wide : launch_walk_philox_f64_wide)(a, field, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 WalkMode walk_mode(const WalkArgs &a, int field, int rng) {
@@ -22,15 +29,19 @@ WalkMode walk_mode(const WalkArgs &a, int field, int rng) {
 }
 
 hipError_t launch_walk_batch(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                             uint32_t spl, int views, int rng, int field, int prec, bool cross, int addr,
+                             uint32_t spl, int views, int rng, int field, int prec, int variant, int addr,
                              size_t lds, hipStream_t s) {
     if (n_slots == 0) return hipSuccess;
     if (n_slots % 8 || threads == 0 || threads > 256 || threads % 64 || spl == 0) return hipErrorInvalidValue;
-    if (rng == 1)
-        return launch_walk_batch_replay(items, chunks, n_slots, threads, spl, views, field, prec, cross, addr, lds, s);
-    if (rng == 0)
-        return launch_walk_batch_philox(items, chunks, n_slots, threads, spl, views, field, prec, cross, addr, lds, s);
-    return hipErrorInvalidValue;
+    const bool half = field >= 2;
+    if (rng < 0 || rng > 1 || prec < 0 || prec > 2 || (prec == 2 && half)) return hipErrorInvalidValue;
+    const auto launch =
+        prec == 2 ? (rng ? launch_walk_batch_replay_f64_wide : launch_walk_batch_philox_f64_wide)
+        : prec == 1 ? (rng ? (half ? launch_walk_batch_replay_kahan_half : launch_walk_batch_replay_kahan_wide)
+                           : (half ? launch_walk_batch_philox_kahan_half : launch_walk_batch_philox_kahan_wide))
+                    : (rng ? (half ? launch_walk_batch_replay_f32_half : launch_walk_batch_replay_f32_wide)
+                           : (half ? launch_walk_batch_philox_f32_half : launch_walk_batch_philox_f32_wide));
+    return launch(items, chunks, n_slots, threads, spl, views, field, variant, addr, lds, s);
 }
 
 __global__ void zero_u64_kernel(unsigned long long *p, int n) {

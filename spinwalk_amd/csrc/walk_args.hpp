@@ -166,6 +166,7 @@ struct WalkArgs {
     uint32_t        n_sub;
     uint32_t        tissue_lds;   // 1: each workgroup copies the tissue tables to LDS (tissue_lds_words)
     uint32_t        pairs;        // 1: a single production walk takes two attempts per trip of its step loop
+    uint32_t        closed;       // 1: no crossing probability between two tissues is above 0
     uint32_t        super_blocks; // 1: the packed records are grouped in super-blocks (kSuper)
     const RfPulse  *rf;           // [n_rf]; entry 0 unused (excitation)
     uint32_t        n_rf;
@@ -207,6 +208,18 @@ struct WalkArgs {
 constexpr uint32_t kTissueLdsMax = 16;
 SW_HD_INLINE uint32_t tissue_lds_words(const WalkArgs &a) {
     return a.tissue_lds ? a.n_sub * a.n_sub + 5 * a.n_sub : 0u;
+}
+
+// The kernel a walk takes.  Production walks of a scan with one TR, and those that
+// record trajectories, take the step loop of walk_prod.hpp; scans with dummy TRs
+// keep the general loop, whose TR set-up is the cheaper one (the 1000^3 bSSFP
+// batch of 100 dummy TRs: 117.2 ms against 121.6 ms; the FoV sweep, one TR each:
+// 120.4 against 118.7 ms).  The general loop is compiled per boundary rule.
+enum Variant : int { VARIANT_PLAIN = 0, VARIANT_CROSS = 1, VARIANT_ONE_TR = 2, VARIANT_TRAJ = 3, VARIANTS = 4 };
+SW_HD_INLINE int walk_variant(const WalkArgs &a, bool replay) {
+    if (!replay && a.record_traj) return VARIANT_TRAJ;
+    if (!replay && a.n_dummy == 0) return VARIANT_ONE_TR;
+    return a.cross_fov ? VARIANT_CROSS : VARIANT_PLAIN;
 }
 
 // An item of the fused batched walk: view 0 is `a`, views 1..n_views-1 are xv;

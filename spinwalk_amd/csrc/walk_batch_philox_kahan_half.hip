@@ -1,0 +1,4 @@
+// The walk kernels of one family (walk_launch.hpp): Philox4x32-10 draws, batched.
+#include "walk_family.hpp"
+
+SW_BATCH_FAMILY(philox_kahan_half, PhiloxRng, PhaseKahan, launch_batch_half)

@@ -1,8 +1,6 @@
 // walk_impl.hpp -- the per-spin Monte-Carlo walk for gfx950 (MI355X): device
-// code and launch templates, instantiated by walk_replay.hip (replayed draws)
-// and walk_philox.hip / walk_batch_philox.hip (production draws), so that the
-// kernel families compile in parallel.
-//
+// code and launch templates, instantiated by walk_*.hip, one kernel family each
+// (walk_family.hpp), so that the families compile in parallel.
 //
 // One lane walks one spin through the whole sequence, as the reference kernel
 // does (src/sim/kernels.cu:55-63 maps thread -> spin and runs sim()), but the
@@ -166,7 +164,7 @@ struct RecF32 {                          // {float field_T, uint32 label}
     static constexpr bool kMixedLayout = false;
     using T = uint2;
     __device__ static uint32_t label(T r) { return r.y; }
-    template <class R> __device__ static R field(const WalkArgs &a, T r) {
+    template <class R, class A> __device__ static R field(const A &a, T r) {
         if (sizeof(R) == 8) return (R)((double)__uint_as_float(r.x) * a.t2d_f64);
         return (R)(__uint_as_float(r.x) * a.t2d);
     }
@@ -177,7 +175,7 @@ struct RecNone {                         // label only: {0, uint8 label, pad}
     static constexpr bool kMixedLayout = false;
     using T = uint32_t;
     __device__ static uint32_t label(T r) { return r >> 16; }
-    template <class R> __device__ static R field(const WalkArgs &, T) { return (R)0; }
+    template <class R, class A> __device__ static R field(const A &, T) { return (R)0; }
 };
 // The 16-bit fields: packed 3-byte records {uint8 label, 16-bit field} in
 // bricks of 3 x 3 x 4 voxels (kPack16).  A record index is the byte offset of
@@ -196,17 +194,17 @@ struct Rec16 {
     }
 };
 struct RecF16 : Rec16 {                  // fp16 field_T / half_scale
-    template <class R> __device__ static R field(const WalkArgs &a, T r) {
+    template <class R, class A> __device__ static R field(const A &a, T r) {
         return (R)(__half2float(__ushort_as_half((unsigned short)bits(r))) * a.h2d);
     }
 };
 struct RecQ16 : Rec16 {                  // int16 rint(field_T / q_scale)
-    template <class R> __device__ static R field(const WalkArgs &a, T r) {
+    template <class R, class A> __device__ static R field(const A &a, T r) {
         return (R)((float)(int32_t)(int16_t)(uint16_t)bits(r) * a.h2d);
     }
 };
 struct RecBF16 : Rec16 {                 // bf16 field_T / half_scale
-    template <class R> __device__ static R field(const WalkArgs &a, T r) {
+    template <class R, class A> __device__ static R field(const A &a, T r) {
         return (R)(__uint_as_float(bits(r) << 16) * a.h2d);
     }
 };
@@ -222,7 +220,7 @@ struct RecF32P {
     static constexpr PackShape pack = kPackF32;
     using T = uint2;                     // the 8 bytes loaded: x = bytes 0-3, y = bytes 4-7
     __device__ static uint32_t label(T r) { return r.x & 0xFFu; }
-    template <class R> __device__ static R field(const WalkArgs &a, T r) {
+    template <class R, class A> __device__ static R field(const A &a, T r) {
         uint2 f;
         f.x = __builtin_amdgcn_alignbit(r.y, r.x, 8);                      // bytes 1-4
         return RecF32::field<R>(a, f);
@@ -243,7 +241,7 @@ struct RecF32S {
     static constexpr PackShape pack = kSoaF32;
     using T = uint2;                     // {field bits, label}, as RecF32
     __device__ static uint32_t label(T r) { return r.y; }
-    template <class R> __device__ static R field(const WalkArgs &a, T r) { return RecF32::field<R>(a, r); }
+    template <class R, class A> __device__ static R field(const A &a, T r) { return RecF32::field<R>(a, r); }
     template <bool IDX32, class I> __device__ static T load(const void *base, I off) {
         const I foff = off + (I)3 * (off & (I)127);                       // field - nvox, as an offset
         T r;
@@ -252,6 +250,8 @@ struct RecF32S {
         return r;
     }
 };
+
+template <class T> struct TypeIs { using type = T; };
 
 // A packed record type whose arrays, in one batch, come in both layouts: the
 // 64-bit lookups read each item's super_blocks flag (ADDR_64_MIXED).
@@ -371,8 +371,8 @@ extern __shared__ uint32_t axis_tab[];
 // x (nb_y nb_z SL 128 bytes, checked below 2^32 on the host) and y fit 32 bits:
 // the divisions run in 32-bit arithmetic and each part takes one 32 x 32 -> 64
 // multiply-add in the 64-bit mode.
-template <class Rec, int SX, int SY, int SZ, class I>
-__device__ __forceinline__ I pack_part_of(const WalkArgs &a, int axis, I i_) {
+template <class Rec, int SX, int SY, int SZ, class I, class A>
+__device__ __forceinline__ I pack_part_of(const A &a, int axis, I i_) {
     constexpr PackShape S = Rec::pack;
     constexpr uint32_t SL = SX * SY * SZ;
     const uint32_t i = (uint32_t)i_;
@@ -392,14 +392,14 @@ __device__ __forceinline__ I pack_part_of(const WalkArgs &a, int axis, I i_) {
 }
 
 // The array's layout is uniform across the launch: a scalar branch picks the form.
-template <class Rec, class I>
-__device__ __forceinline__ I pack_part(const WalkArgs &a, int axis, I i) {
+template <class Rec, class I, class A>
+__device__ __forceinline__ I pack_part(const A &a, int axis, I i) {
     if (a.super_blocks) return pack_part_of<Rec, kSuper.sx, kSuper.sy, kSuper.sz>(a, axis, i);
     return pack_part_of<Rec, 1, 1, 1>(a, axis, i);
 }
 
-template <class Rec>
-__device__ __forceinline__ uint32_t axis_entry(const WalkArgs &a, uint32_t i) {
+template <class Rec, class A>
+__device__ __forceinline__ uint32_t axis_entry(const A &a, uint32_t i) {
     const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny;
     if constexpr (Rec::kPacked) {
         if (i < nx) return pack_part<Rec, uint32_t>(a, 0, i);
@@ -418,8 +418,8 @@ __device__ __forceinline__ uint32_t axis_entry(const WalkArgs &a, uint32_t i) {
     }
 }
 
-template <class Rec, bool IDX32>
-__device__ __forceinline__ uint64_t record_of(const WalkArgs &a, uint64_t ix, uint64_t iy, uint64_t iz) {
+template <class Rec, bool IDX32, class A>
+__device__ __forceinline__ uint64_t record_of(const A &a, uint64_t ix, uint64_t iy, uint64_t iz) {
     if (IDX32) {
         const uint32_t nx = (uint32_t)a.nx, nxy = nx + (uint32_t)a.ny;
         return axis_tab[(uint32_t)ix] + axis_tab[nx + (uint32_t)iy] + axis_tab[nxy + (uint32_t)iz];
@@ -452,14 +452,27 @@ __device__ __forceinline__ uint32_t cvt_i32_sat(double v) {
     return r;
 }
 
-// A voxel some of whose scaled coordinates lie outside [0, n): the reference's
-// int64 arithmetic on the truncated coordinates.
-template <class Rec, bool IDX32>
-__device__ __forceinline__ Vox<IDX32> locate_outside(const WalkArgs &a, double vx, double vy, double vz) {
+// The subscripts of the voxel that the reference's int64 arithmetic finds for
+// scaled coordinates some of which lie outside [0, n); false outside the volume.
+template <class A>
+__device__ __forceinline__ bool wrapped_subscripts(const A &a, double vx, double vy, double vz, uint32_t s[3]) {
+    constexpr double kLim = 9.2e18;   // beyond int64 the conversion is undefined; treat as outside
+    if (!(fabs(vx) < kLim && fabs(vy) < kLim && fabs(vz) < kLim)) return false;
+    const int64_t jx = (int64_t)vx, jy = (int64_t)vy, jz = (int64_t)vz;
+    const int64_t ind = jx * a.nz * a.ny + jy * a.nz + jz;     // kernels.cuh:53-60
+    if (ind < 0 || ind >= a.matrix_length) return false;        // kernels.cu:141
+    const uint64_t u = (uint64_t)ind, nz = (uint64_t)a.nz, ny = (uint64_t)a.ny;
+    s[0] = (uint32_t)(u / (nz * ny)); s[1] = (uint32_t)((u / nz) % ny); s[2] = (uint32_t)(u % nz);   // each in range
+    return true;
+}
+
+// A voxel some of whose scaled coordinates lie outside [0, n): its record.
+template <class Rec, bool IDX32, class A>
+__device__ __forceinline__ Vox<IDX32> locate_outside(const A &a, double vx, double vy, double vz) {
     Vox<IDX32> v;
     v.ok = false;
     v.rec = 0;
-    constexpr double kLim = 9.2e18;   // beyond int64 the conversion is undefined; treat as outside
+    constexpr double kLim = 9.2e18;
     if (!(fabs(vx) < kLim && fabs(vy) < kLim && fabs(vz) < kLim)) return v;
     const int64_t jx = (int64_t)vx, jy = (int64_t)vy, jz = (int64_t)vz;
     const int64_t ind = jx * a.nz * a.ny + jy * a.nz + jz;     // kernels.cuh:53-60
@@ -606,10 +619,10 @@ struct PosVox {
         }
         __device__ bool moves() const { return d[0] == d[0]; }
     };
-    __device__ static T start(const WalkArgs &a, float x0, int i) { return x0 * a.s2gf[i]; }
-    __device__ static float metres(const WalkArgs &a, T p, int i) { return p * a.vsf[i]; }
-    template <class Rec, bool IDX32>
-    __device__ static Vox<IDX32> find(const WalkArgs &a, const T p[3]) {
+    template <class A> __device__ static T start(const A &a, float x0, int i) { return x0 * a.s2gf[i]; }
+    template <class A> __device__ static float metres(const A &a, T p, int i) { return p * a.vsf[i]; }
+    template <class Rec, bool IDX32, class A>
+    __device__ static Vox<IDX32> find(const A &a, const T p[3]) {
         const uint32_t ix = cvt_i32_sat_f(p[0]), iy = cvt_i32_sat_f(p[1]), iz = cvt_i32_sat_f(p[2]);
         if (ix < (uint32_t)a.nx && iy < (uint32_t)a.ny && iz < (uint32_t)a.nz) {
             Vox<IDX32> v;
@@ -653,8 +666,8 @@ struct PosVox {
     }
     // The gradient phase of a step from the position in metres: in double for the
     // FP64 walk, in float (g2d = 1e-3 dt 1e-6 gamma rad2deg) for the others.
-    template <class Phase>
-    __device__ static void add_grad(Phase &ph, const WalkArgs &a, float Gx, float Gy, float Gz, const T p[3]) {
+    template <class Phase, class A>
+    __device__ static void add_grad(Phase &ph, const A &a, float Gx, float Gy, float Gz, const T p[3]) {
         if constexpr (sizeof(typename Phase::R) == 8) {
             const double x = (double)p[0] * a.vs[0], y = (double)p[1] * a.vs[1], z = (double)p[2] * a.vs[2];
             ph.add_grad((Gx * x + Gy * y + Gz * z) * 1e-3 * a.timestep_us * 1e-6 * kGamma * kRad2Deg);
@@ -753,6 +766,14 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
     }
     return ((uint64_t)hi << 32) | lo;
 }
+
+}  // namespace
+}  // namespace sw
+
+#include "walk_prod.hpp"
+
+namespace sw {
+namespace {
 
 template <class Rng, class Rec, class Phase, bool CROSS, bool IDX32>
 __device__ int walk_spin(const WalkArgs &a, uint32_t li, uint64_t &n_acc, uint32_t &n_rej) {
@@ -952,7 +973,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, uint32_t t0, uint3
         if (t < a.n_local) {
             const uint32_t li = a.order ? a.order[t] : t;
             int st;
-            if constexpr (Rng::kReplay || !PAIRS) st = walk_spin<Rng, Rec, Phase, CROSS, IDX32>(a, li, n_acc, n_rej);
+            if constexpr (!PAIRS) st = walk_spin<Rng, Rec, Phase, CROSS, IDX32>(a, li, n_acc, n_rej);
             else st = walk_spin_pairs<Rec, Phase, CROSS, IDX32, 1>(a, nullptr, li, n_acc, n_rej);
             lost += (st == ST_LOST);
             exh += (st == ST_EXHAUSTED);
@@ -1506,6 +1527,16 @@ void walk_kernel(const WalkArgs a) {
     walk_block<Rng, Rec, Phase, CROSS, IDX32, PAIRS>(a, lb * blockDim.x);
 }
 
+// The production walk with one attempt per trip (walk_prod.hpp).  The arguments
+// are read where they are passed, in the constant address space.
+template <class Rec, class Phase, bool IDX32, bool ONE_TR, bool TRAJ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SW_WALK_WAVES_PER_EU)))
+void walk_prod_kernel(const WalkArgs) {
+    const uint32_t per = gridDim.x / 8, b = blockIdx.x;
+    const uint32_t lb = (b % 8) * per + b / 8;
+    prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>((ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), nullptr, 1, lb * blockDim.x, 1);
+}
+
 // The batched walk: block b takes the chunk at slot (b mod 8) * (grid / 8) + b / 8
 // of the chunk table, i.e. XCD k works through slots [k * grid/8, (k+1) * grid/8)
 // in order.  The host lays each XCD's slots out longest tile first, so the long
@@ -1536,6 +1567,21 @@ void walk_batch_kernel(const void *__restrict__ items, const BatchChunk *__restr
     } else {
         const FusedArgs &f = ((const FusedArgs *)items)[c.item];
         walk_block_views<Rng, Rec, Phase, CROSS, IDX32, NV>(f.a, f.xv, f.n_views, c.first, spl);
+    }
+}
+
+// The production form of walk_batch_kernel.
+template <class Rec, class Phase, bool IDX32, int NV, bool ONE_TR, bool TRAJ>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(walk_waves_per_eu<Phase, NV>())))
+void walk_batch_prod_kernel(const void *__restrict__ items, const BatchChunk *__restrict__ chunks, uint32_t spl) {
+    const uint32_t per = gridDim.x / 8, b = blockIdx.x;
+    const BatchChunk c = chunks[(b % 8) * per + b / 8];
+    if (c.item == kNoItem) return;                    // padding slot (uniform across the block)
+    if constexpr (NV == 1) {
+        prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>((ArgsPtr)((const WalkArgs *)items + c.item), nullptr, 1, c.first, spl);
+    } else {
+        const auto *f = (const __attribute__((address_space(4))) FusedArgs *)((const FusedArgs *)items + c.item);
+        prod_block<Rec, Phase, IDX32, NV, ONE_TR, TRAJ>(&f->a, f->xv, f->n_views, c.first, spl);
     }
 }
 
@@ -1577,44 +1623,72 @@ hipError_t launch_fp_loop(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 bloc
     return hipGetLastError();
 }
 
-template <class Rng, class F, class P>
-hipError_t launch_fp(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
-    if constexpr (!Rng::kReplay) {
-        if (a.pairs) return launch_fp_loop<Rng, F, P, true>(a, s, grid, block);
-    }
-    return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
-}
-
-template <class Rng, class F, class P, int NV>
-hipError_t launch_batch_nv(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                           uint32_t spl, bool cross, int addr, size_t lds, hipStream_t s) {
-    const dim3 grid(n_slots), block(threads);
+template <class F, class P, bool ONE_TR, bool TRAJ>
+hipError_t launch_prod(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
+    const WalkMode m = mode_of<F>(a);
     if constexpr (F::kPacked) {
-        if (addr == ADDR_64_MIXED) {
-            if (cross) hipLaunchKernelGGL((walk_batch_kernel<Rng, MixedLayout<F>, P, true, false, NV>), grid, block, lds, s, items, chunks, spl);
-            else       hipLaunchKernelGGL((walk_batch_kernel<Rng, MixedLayout<F>, P, false, false, NV>), grid, block, lds, s, items, chunks, spl);
-            return hipGetLastError();
-        }
+        if (!m.idx32 && a.super_blocks) return hipErrorInvalidValue;   // super-blocks always fit the 32-bit mode
     }
-    const bool idx32 = addr == ADDR_32;
-    if (cross) {
-        if (idx32) hipLaunchKernelGGL((walk_batch_kernel<Rng, F, P, true, true, NV>), grid, block, lds, s, items, chunks, spl);
-        else       hipLaunchKernelGGL((walk_batch_kernel<Rng, F, P, true, false, NV>), grid, block, lds, s, items, chunks, spl);
-    } else {
-        if (idx32) hipLaunchKernelGGL((walk_batch_kernel<Rng, F, P, false, true, NV>), grid, block, lds, s, items, chunks, spl);
-        else       hipLaunchKernelGGL((walk_batch_kernel<Rng, F, P, false, false, NV>), grid, block, lds, s, items, chunks, spl);
-    }
+    if (m.idx32) hipLaunchKernelGGL((walk_prod_kernel<F, P, true, ONE_TR, TRAJ>), grid, block, m.lds, s, a);
+    else         hipLaunchKernelGGL((walk_prod_kernel<F, P, false, ONE_TR, TRAJ>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-// views: 1, or kMaxViews for fused items (FP32 and Kahan phases only).
+template <class Rng, class F, class P>
+hipError_t launch_fp(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
+    if constexpr (Rng::kReplay) {
+        return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
+    } else {
+        if (a.pairs) return launch_fp_loop<Rng, F, P, true>(a, s, grid, block);
+        switch (walk_variant(a, false)) {
+        case VARIANT_TRAJ: return launch_prod<F, P, false, true>(a, s, grid, block);
+        case VARIANT_ONE_TR: return launch_prod<F, P, true, false>(a, s, grid, block);
+        default: return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
+        }
+    }
+}
+
+template <class Rng, class F, class P, int NV, int VARIANT>
+hipError_t launch_batch_nv(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
+                           uint32_t spl, int addr, size_t lds, hipStream_t s) {
+    const dim3 grid(n_slots), block(threads);
+    auto go = [&](auto idx32, auto rec) {
+        constexpr bool IDX32 = decltype(idx32)::value;
+        using Rec = typename decltype(rec)::type;
+        if constexpr (VARIANT == VARIANT_ONE_TR || VARIANT == VARIANT_TRAJ)
+            hipLaunchKernelGGL((walk_batch_prod_kernel<Rec, P, IDX32, NV, VARIANT == VARIANT_ONE_TR, VARIANT == VARIANT_TRAJ>),
+                               grid, block, lds, s, items, chunks, spl);
+        else
+            hipLaunchKernelGGL((walk_batch_kernel<Rng, Rec, P, VARIANT == VARIANT_CROSS, IDX32, NV>), grid, block, lds, s,
+                               items, chunks, spl);
+        return hipGetLastError();
+    };
+    if (addr == ADDR_32) return go(std::true_type(), TypeIs<F>());
+    if constexpr (F::kPacked) {
+        if (addr == ADDR_64_MIXED) return go(std::false_type(), TypeIs<MixedLayout<F>>());
+    }
+    return go(std::false_type(), TypeIs<F>());
+}
+
+template <class Rng, class F, class P, int NV>
+hipError_t launch_batch_variant(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
+                                uint32_t spl, int variant, int addr, size_t lds, hipStream_t s) {
+    if constexpr (!Rng::kReplay) {
+        if (variant == VARIANT_ONE_TR) return launch_batch_nv<Rng, F, P, NV, VARIANT_ONE_TR>(items, chunks, n_slots, threads, spl, addr, lds, s);
+        if (variant == VARIANT_TRAJ) return launch_batch_nv<Rng, F, P, NV, VARIANT_TRAJ>(items, chunks, n_slots, threads, spl, addr, lds, s);
+    }
+    if (variant == VARIANT_CROSS) return launch_batch_nv<Rng, F, P, NV, VARIANT_CROSS>(items, chunks, n_slots, threads, spl, addr, lds, s);
+    if (variant == VARIANT_PLAIN) return launch_batch_nv<Rng, F, P, NV, VARIANT_PLAIN>(items, chunks, n_slots, threads, spl, addr, lds, s);
+    return hipErrorInvalidValue;
+}
+
 template <class Rng, class F, class P>
 hipError_t launch_batch_fp(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                           uint32_t spl, int views, bool cross, int addr, size_t lds, hipStream_t s) {
-    if (views == 1) return launch_batch_nv<Rng, F, P, 1>(items, chunks, n_slots, threads, spl, cross, addr, lds, s);
+                           uint32_t spl, int views, int variant, int addr, size_t lds, hipStream_t s) {
+    if (views == 1) return launch_batch_variant<Rng, F, P, 1>(items, chunks, n_slots, threads, spl, variant, addr, lds, s);
     if constexpr (sizeof(typename P::R) == 4) {
         if (views == kMaxViews)
-            return launch_batch_nv<Rng, F, P, kMaxViews>(items, chunks, n_slots, threads, spl, cross, addr, lds, s);
+            return launch_batch_variant<Rng, F, P, kMaxViews>(items, chunks, n_slots, threads, spl, variant, addr, lds, s);
     }
     return hipErrorInvalidValue;
 }
@@ -1628,63 +1702,44 @@ hipError_t launch_batch_fp(const void *items, const BatchChunk *chunks, uint32_t
 template <class Rng> using RecF32Batch = typename std::conditional<Rng::kReplay, RecF32, RecF32P>::type;
 template <class Rng> using RecF32Single = typename std::conditional<Rng::kReplay, RecF32, RecF32S>::type;
 
-template <class Rng>
-hipError_t launch_batch_rng(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                            uint32_t spl, int views, int field, int prec, bool cross, int addr, size_t lds,
-                            hipStream_t s) {
-    if (prec == 2) {
-        if (field == 0) return launch_batch_fp<Rng, RecNone, PhaseF64>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 1) return launch_batch_fp<Rng, RecF32Batch<Rng>, PhaseF64>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-    } else if (prec == 1) {
-        if (field == 0) return launch_batch_fp<Rng, RecNone, PhaseKahan>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 1) return launch_batch_fp<Rng, RecF32Batch<Rng>, PhaseKahan>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 2) return launch_batch_fp<Rng, RecF16, PhaseKahan>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 3) return launch_batch_fp<Rng, RecBF16, PhaseKahan>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 4) return launch_batch_fp<Rng, RecQ16, PhaseKahan>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-    } else if (prec == 0) {
-        if (field == 0) return launch_batch_fp<Rng, RecNone, PhaseF32>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 1) return launch_batch_fp<Rng, RecF32Batch<Rng>, PhaseF32>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 2) return launch_batch_fp<Rng, RecF16, PhaseF32>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 3) return launch_batch_fp<Rng, RecBF16, PhaseF32>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-        if (field == 4) return launch_batch_fp<Rng, RecQ16, PhaseF32>(items, chunks, n_slots, threads, spl, views, cross, addr, lds, s);
-    }
+// The families of kernels, one translation unit each: phase P over the float32
+// field or none (wide), or over the 16-bit fields.
+template <class Rng, class P>
+hipError_t launch_batch_wide(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
+                             uint32_t spl, int views, int field, int variant, int addr, size_t lds, hipStream_t s) {
+    if (field == 0) return launch_batch_fp<Rng, RecNone, P>(items, chunks, n_slots, threads, spl, views, variant, addr, lds, s);
+    if (field == 1) return launch_batch_fp<Rng, RecF32Batch<Rng>, P>(items, chunks, n_slots, threads, spl, views, variant, addr, lds, s);
+    return hipErrorInvalidValue;
+}
+template <class Rng, class P>
+hipError_t launch_batch_half(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
+                             uint32_t spl, int views, int field, int variant, int addr, size_t lds, hipStream_t s) {
+    if (field == 2) return launch_batch_fp<Rng, RecF16, P>(items, chunks, n_slots, threads, spl, views, variant, addr, lds, s);
+    if (field == 3) return launch_batch_fp<Rng, RecBF16, P>(items, chunks, n_slots, threads, spl, views, variant, addr, lds, s);
+    if (field == 4) return launch_batch_fp<Rng, RecQ16, P>(items, chunks, n_slots, threads, spl, views, variant, addr, lds, s);
     return hipErrorInvalidValue;
 }
 
-template <class Rng>
-hipError_t launch_rng(const WalkArgs &a, int field, int prec, hipStream_t s) {
+template <class Rng, class P>
+hipError_t launch_wide(const WalkArgs &a, int field, hipStream_t s) {
     const uint32_t nb = (a.n_local + 255) / 256;
     if (nb == 0) return hipSuccess;
     const dim3 block(256), grid((nb + 7) / 8 * 8);
-    if (prec == 2) {
-        if (field == 0) return launch_fp<Rng, RecNone, PhaseF64>(a, s, grid, block);
-        if (field == 1) return launch_fp<Rng, RecF32Single<Rng>, PhaseF64>(a, s, grid, block);
-    } else if (prec == 1) {
-        if (field == 0) return launch_fp<Rng, RecNone, PhaseKahan>(a, s, grid, block);
-        if (field == 1) return launch_fp<Rng, RecF32Single<Rng>, PhaseKahan>(a, s, grid, block);
-        if (field == 2) return launch_fp<Rng, RecF16, PhaseKahan>(a, s, grid, block);
-        if (field == 3) return launch_fp<Rng, RecBF16, PhaseKahan>(a, s, grid, block);
-        if (field == 4) return launch_fp<Rng, RecQ16, PhaseKahan>(a, s, grid, block);
-    } else if (prec == 0) {
-        if (field == 0) return launch_fp<Rng, RecNone, PhaseF32>(a, s, grid, block);
-        if (field == 1) return launch_fp<Rng, RecF32Single<Rng>, PhaseF32>(a, s, grid, block);
-        if (field == 2) return launch_fp<Rng, RecF16, PhaseF32>(a, s, grid, block);
-        if (field == 3) return launch_fp<Rng, RecBF16, PhaseF32>(a, s, grid, block);
-        if (field == 4) return launch_fp<Rng, RecQ16, PhaseF32>(a, s, grid, block);
-    }
+    if (field == 0) return launch_fp<Rng, RecNone, P>(a, s, grid, block);
+    if (field == 1) return launch_fp<Rng, RecF32Single<Rng>, P>(a, s, grid, block);
+    return hipErrorInvalidValue;
+}
+template <class Rng, class P>
+hipError_t launch_half(const WalkArgs &a, int field, hipStream_t s) {
+    const uint32_t nb = (a.n_local + 255) / 256;
+    if (nb == 0) return hipSuccess;
+    const dim3 block(256), grid((nb + 7) / 8 * 8);
+    if (field == 2) return launch_fp<Rng, RecF16, P>(a, s, grid, block);
+    if (field == 3) return launch_fp<Rng, RecBF16, P>(a, s, grid, block);
+    if (field == 4) return launch_fp<Rng, RecQ16, P>(a, s, grid, block);
     return hipErrorInvalidValue;
 }
 
 }  // namespace
-
-// Launchers of the kernel families (one translation unit each).
-hipError_t launch_walk_replay(const WalkArgs &a, int field, int prec, hipStream_t s);
-hipError_t launch_walk_philox(const WalkArgs &a, int field, int prec, hipStream_t s);
-hipError_t launch_walk_batch_replay(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                                    uint32_t spl, int views, int field, int prec, bool cross, int addr, size_t lds,
-                                    hipStream_t s);
-hipError_t launch_walk_batch_philox(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                                    uint32_t spl, int views, int field, int prec, bool cross, int addr, size_t lds,
-                                    hipStream_t s);
 
 }  // namespace sw

@@ -21,12 +21,25 @@ WalkMode walk_mode(const WalkArgs &a, int field, int rng);
 // one workgroup of `threads` lanes (64, 128 or 256) per chunk of threads * spl
 // spins (each lane walks spl spins, one after the other):
 // items[] (WalkArgs, or FusedArgs when views == kMaxViews; prec 0 or 1 only)
-// and chunks[] in device memory; every item shares rng, field, prec, cross and
-// the address mode (AddrMode; ADDR_32 with `lds` bytes covering every item's
-// tables).
+// and chunks[] in device memory; every item shares rng, field, prec, the variant
+// (walk_variant) and the address mode (AddrMode; ADDR_32 with `lds` bytes covering every item's tables).
 hipError_t launch_walk_batch(const void *items, const BatchChunk *chunks, uint32_t n_slots, uint32_t threads,
-                             uint32_t spl, int views, int rng, int field, int prec, bool cross, int addr,
+                             uint32_t spl, int views, int rng, int field, int prec, int variant, int addr,
                              size_t lds, hipStream_t s);
+
+// The launchers of the kernel families (walk_impl.hpp), one translation unit each:
+// replayed or Philox draws; FP32, Kahan or FP64 phase; float32 field or none
+// (wide), or a 16-bit field (half).
+#define SW_FAMILIES(X) \
+    X(replay_f32_wide) X(replay_f32_half) X(replay_kahan_wide) X(replay_kahan_half) X(replay_f64_wide) \
+    X(philox_f32_wide) X(philox_f32_half) X(philox_kahan_wide) X(philox_kahan_half) X(philox_f64_wide)
+#define SW_DECLARE_FAMILY(name)                                                                                  \
+    hipError_t launch_walk_##name(const WalkArgs &a, int field, hipStream_t s);                                  \
+    hipError_t launch_walk_batch_##name(const void *items, const BatchChunk *chunks, uint32_t n_slots,           \
+                                        uint32_t threads, uint32_t spl, int views, int field, int variant,       \
+                                        int addr, size_t lds, hipStream_t s);
+SW_FAMILIES(SW_DECLARE_FAMILY)
+#undef SW_DECLARE_FAMILY
 
 // Production draws of spins [spin0, spin0+n_spins), attempts [0, n_att).
 hipError_t launch_philox_draws(uint64_t seed, uint32_t spin0, uint32_t n_spins, uint32_t n_att,
