@@ -13,6 +13,7 @@
 #include <cstring>
 #include <math.h>
 #include <memory>
+#include <mutex>
 #include <random>
 #include <string>
 #include <thread>
@@ -36,11 +37,70 @@ thread_local std::string g_tls_error;
 
 }  // namespace
 
+// Device memory of phantoms that are gone, kept for the next ones: a program that
+// sweeps over geometries makes and drops a phantom per step, and taking and giving
+// back its memory each time cost more than preparing it (256^3, float32: 1.2 ms of
+// a 2.5 ms step; at higher rates the driver stalls whole calls by 10 ms).  At
+// most kBlocks blocks of kBytes in all; a block serves a phantom of its size or
+// down to half of it.  Given back when an allocation does not fit beside them and
+// with the engine; a phantom that outlives its engine frees its own.  Shared by
+// the engine and its phantoms, which may be destroyed from any thread.
+struct PhantomPool {
+    static constexpr size_t kBlocks = 4, kBytes = 2ull << 30;
+    std::mutex mu;
+    bool open = true;
+    std::vector<std::pair<void *, size_t>> kept;
+    void *take(size_t bytes, size_t *got) {
+        std::lock_guard<std::mutex> lock(mu);
+        for (size_t i = 0; i < kept.size(); i++)
+            if (kept[i].second >= bytes && kept[i].second / 2 <= bytes) {
+                void *p = kept[i].first;
+                *got = kept[i].second;
+                kept.erase(kept.begin() + i);
+                return p;
+            }
+        return nullptr;
+    }
+    // The device has finished with p.
+    void put(void *p, size_t bytes) {
+        std::vector<void *> drop;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            size_t sum = bytes;
+            for (const auto &k : kept) sum += k.second;
+            if (!open || bytes > kBytes) drop.push_back(p);
+            else {
+                while (!kept.empty() && (kept.size() >= kBlocks || sum > kBytes)) {   // the oldest first
+                    sum -= kept.front().second;
+                    drop.push_back(kept.front().first);
+                    kept.erase(kept.begin());
+                }
+                kept.push_back({p, bytes});
+            }
+        }
+        for (void *d : drop) (void)hipFree(d);
+    }
+    void release(bool close) {
+        std::vector<std::pair<void *, size_t>> drop;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            drop.swap(kept);
+            if (close) open = false;
+        }
+        for (const auto &k : drop) (void)hipFree(k.first);
+    }
+    bool empty() {
+        std::lock_guard<std::mutex> lock(mu);
+        return kept.empty();
+    }
+};
+
 struct sw_engine {
+    std::shared_ptr<PhantomPool> pool = std::make_shared<PhantomPool>();
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
-    unsigned long long *d_counters = nullptr;   // 4 x u64
+    unsigned long long *d_counters = nullptr;   // 4 x u64, then 1 for a phantom's statistics
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // scratch reused across calls
     void *d_sort = nullptr; size_t sort_bytes = 0;
@@ -73,6 +133,10 @@ struct sw_phantom {
     float q_scale = 1.f;             // int16 records hold rint(field_T / q_scale)
     uint32_t n_labels = 0;
     bool has_field = false;
+    // the phantom's device memory: every array below is a slice of it
+    void *arena = nullptr;
+    size_t arena_bytes = 0;
+    std::shared_ptr<PhantomPool> pool;
     // bricked voxel records gathered by the walk (walk_args.hpp)
     void *rec[5] = {};               // by SW_FIELD_*: none (label only), f32, f16, bf16, q16
     void *rec_packed = nullptr;      // float32 packed 5-byte records (production batches)
@@ -202,6 +266,10 @@ int ensure_exc(sw_engine *e, sw_sequence *q, const sw_params *p, hipStream_t s) 
 int check_free_memory(sw_engine *e, size_t bytes) {   // device_helper.cu:78-101
     size_t fr = 0, tot = 0;
     SW_HIP(e, hipMemGetInfo(&fr, &tot));
+    if (bytes > fr && !e->pool->empty()) {
+        e->pool->release(false);
+        SW_HIP(e, hipMemGetInfo(&fr, &tot));
+    }
     if (bytes > fr) {
         char b[256];
         snprintf(b, sizeof b, "not enough device memory: need %zu MB, free %zu MB", bytes >> 20, fr >> 20);
@@ -271,7 +339,7 @@ SW_API int sw_engine_create(int device_id, sw_engine **out) {
     if (hipSetDevice(device_id) != hipSuccess) return fail(nullptr, SW_E_HIP, "hipSetDevice failed");
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(nullptr, SW_E_HIP, "hipStreamCreate failed");
-    if (hipMalloc((void **)&e->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess)
+    if (hipMalloc((void **)&e->d_counters, 5 * sizeof(unsigned long long)) != hipSuccess)
         return fail(nullptr, SW_E_HIP, "hipMalloc counters failed");
     if (hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess ||
         hipEventCreateWithFlags(&e->scratch_ev, hipEventDisableTiming) != hipSuccess)
@@ -290,6 +358,7 @@ SW_API void sw_engine_destroy(sw_engine *e) {
     dev_free(e->d_sort);
     dev_free(e->d_order);
     dev_free(e->d_partial);
+    e->pool->release(true);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->scratch_ev) {
@@ -386,16 +455,63 @@ static size_t phantom_bytes(uint64_t n, bool has_field, uint32_t formats) {
     return need;
 }
 
+// Takes the phantom's device memory and lays its arrays out in it.
+static int phantom_alloc(sw_engine *e, sw_phantom *ph, uint32_t formats) {
+    const uint64_t nx = ph->dims[0], ny = ph->dims[1], nz = ph->dims[2];
+    size_t total = 0;
+    std::vector<std::pair<void **, size_t>> slices;
+    auto slice = [&](void **p, size_t bytes) {
+        slices.push_back({p, total});
+        total += (bytes + 4095) & ~(size_t)4095;
+    };
+    slice((void **)&ph->mask, ph->n);
+    if (ph->has_field) slice((void **)&ph->field, ph->n * sizeof(float));
+    for (int f = 0; f <= SW_FIELD_Q16; f++) {
+        const bool want = (f == SW_FIELD_NONE) ? !ph->has_field : (ph->has_field && (formats & (1u << f)));
+        if (!want) continue;
+        if (f == SW_FIELD_F16 || f == SW_FIELD_BF16 || f == SW_FIELD_Q16) {   // packed 3-byte records
+            slice(&ph->rec[f], (size_t)sw::pack_bytes(nx, ny, nz, sw::kPack16, sw::pack_super(nx, ny, nz, sw::kPack16)));
+            continue;
+        }
+        const sw::BrickShape sh = f == SW_FIELD_F32 ? sw::kBrick8 : sw::kBrick4;
+        slice(&ph->rec[f], ((size_t)(sw::brick_count(nx, sh.lbx) * sw::brick_count(ny, sh.lby) * sw::brick_count(nz, sh.lbz))
+                            << (sh.lbx + sh.lby + sh.lbz)) * (f == SW_FIELD_F32 ? 8 : 4));
+        if (f == SW_FIELD_F32) {         // the production walks' copies: packed for batches, SoA for single walks
+            const size_t bytes = (size_t)sw::pack_bytes(nx, ny, nz, sw::kPackF32, sw::pack_super(nx, ny, nz, sw::kPackF32));
+            slice(&ph->rec_packed, bytes);
+            slice(&ph->rec_soa, bytes);
+        }
+    }
+    ph->pool = e->pool;
+    ph->arena = e->pool->take(total, &ph->arena_bytes);
+    if (!ph->arena) {
+        ph->arena_bytes = total;
+        hipError_t he = hipMalloc(&ph->arena, total);
+        if (he != hipSuccess && !e->pool->empty()) {         // again without what the pool holds
+            (void)hipGetLastError();
+            e->pool->release(false);
+            he = hipMalloc(&ph->arena, total);
+        }
+        if (he != hipSuccess) {
+            ph->arena = nullptr;
+            return fail(e, SW_E_HIP, std::string("hipMalloc of a phantom: ") + hipGetErrorString(he));
+        }
+    }
+    for (const auto &x : slices) *x.first = (char *)ph->arena + x.second;
+    return SW_OK;
+}
+
 static int phantom_finish(sw_engine *e, sw_phantom *ph, uint32_t formats) {
     hipStream_t s = e->stream;
     uint32_t st[2] = {0, 0};
     {
-        uint32_t *d_stats = nullptr;
-        SW_HIP(e, hipMalloc((void **)&d_stats, 2 * sizeof(uint32_t)));
-        std::unique_ptr<uint32_t, void (*)(uint32_t *)> guard(d_stats, [](uint32_t *p) { dev_free(p); });
-        SW_HIP(e, hipMemsetAsync(d_stats, 0, 2 * sizeof(uint32_t), s));
+        uint32_t *d_stats = (uint32_t *)(e->d_counters + 4);
+        int rc = scratch_acquire(e, s);
+        if (rc) return rc;
+        SW_HIP(e, sw::launch_zero_u64(e->d_counters + 4, 1, s));
         SW_HIP(e, sw::launch_phantom_stats(ph->mask, ph->field, ph->n, d_stats, s));
         SW_HIP(e, hipMemcpyAsync(st, d_stats, sizeof st, hipMemcpyDeviceToHost, s));
+        if ((rc = scratch_release(e, s))) return rc;
         SW_HIP(e, hipStreamSynchronize(s));
     }
     ph->n_labels = st[0] + 1;                                    // monte_carlo.cu:113
@@ -414,24 +530,20 @@ static int phantom_finish(sw_engine *e, sw_phantom *ph, uint32_t formats) {
     for (int f = 0; f <= SW_FIELD_Q16; f++) {
         const bool want = (f == SW_FIELD_NONE) ? !ph->has_field : (ph->has_field && (formats & (1u << f)));
         if (!want) continue;
-        size_t bytes;
-        if (f == SW_FIELD_F16 || f == SW_FIELD_BF16 || f == SW_FIELD_Q16) {   // packed 3-byte records
-            bytes = (size_t)sw::pack_bytes(nx, ny, nz, sw::kPack16, sw::pack_super(nx, ny, nz, sw::kPack16));
-        } else {
+        if (f == SW_FIELD_F32 || f == SW_FIELD_NONE) {
             const sw::BrickShape sh = f == SW_FIELD_F32 ? sw::kBrick8 : sw::kBrick4;
-            bytes = ((size_t)(sw::brick_count(nx, sh.lbx) * sw::brick_count(ny, sh.lby) * sw::brick_count(nz, sh.lbz))
-                     << (sh.lbx + sh.lby + sh.lbz)) * (f == SW_FIELD_F32 ? 8 : 4);
+            SW_HIP(e, hipMemsetAsync(ph->rec[f], 0, ((size_t)(sw::brick_count(nx, sh.lbx) * sw::brick_count(ny, sh.lby) *
+                                     sw::brick_count(nz, sh.lbz)) << (sh.lbx + sh.lby + sh.lbz)) * (f == SW_FIELD_F32 ? 8 : 4), s));
+        } else {
+            SW_HIP(e, hipMemsetAsync(ph->rec[f], 0, (size_t)sw::pack_bytes(nx, ny, nz, sw::kPack16, sw::pack_super(nx, ny, nz, sw::kPack16)), s));
         }
-        SW_HIP(e, hipMalloc(&ph->rec[f], bytes));
-        SW_HIP(e, hipMemsetAsync(ph->rec[f], 0, bytes, s));
         const int kind = f == SW_FIELD_F32 ? 0 : f == SW_FIELD_F16 ? 1 : f == SW_FIELD_BF16 ? 2 : f == SW_FIELD_Q16 ? 4 : 3;
         SW_HIP(e, sw::launch_records(ph->mask, ph->field, nx, ny, nz, kind,
                                      1.0f / (f == SW_FIELD_Q16 ? ph->q_scale : ph->half_scale), ph->rec[f], s));
         if (f == SW_FIELD_F32) {         // the production walks' copies: packed for batches, SoA for single walks
             const size_t bytes = (size_t)sw::pack_bytes(nx, ny, nz, sw::kPackF32, sw::pack_super(nx, ny, nz, sw::kPackF32));
             for (int soa = 0; soa < 2; soa++) {
-                void *&r = soa ? ph->rec_soa : ph->rec_packed;
-                SW_HIP(e, hipMalloc(&r, bytes));
+                void *r = soa ? ph->rec_soa : ph->rec_packed;
                 SW_HIP(e, hipMemsetAsync(r, 0, bytes, s));
                 SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, soa != 0, r, s));
             }
@@ -457,10 +569,9 @@ static int phantom_create_common(sw_engine *e, const uint8_t *mask, const float 
     int rc = check_free_memory(e, phantom_bytes(ph->n, ph->has_field, formats) + (64u << 20));
     if (rc) return rc;
     hipStream_t s = e->stream;
-    SW_HIP(e, hipMalloc((void **)&ph->mask, ph->n));
+    if ((rc = phantom_alloc(e, ph.get(), formats))) return rc;
     SW_HIP(e, hipMemcpyAsync(ph->mask, mask, ph->n, kind, s));
     if (ph->has_field) {
-        SW_HIP(e, hipMalloc((void **)&ph->field, ph->n * sizeof(float)));
         SW_HIP(e, hipMemcpyAsync(ph->field, field, ph->n * sizeof(float), kind, s));
     }
     SW_HIP(e, hipStreamSynchronize(s));
@@ -483,11 +594,11 @@ SW_API int sw_phantom_create_device(sw_engine *e, const uint8_t *d_mask, const f
 SW_API void sw_phantom_destroy(sw_phantom *ph) {
     if (!ph) return;
     (void)hipSetDevice(ph->device);
-    dev_free(ph->mask);
-    dev_free(ph->field);
-    for (void *r : ph->rec) dev_free(r);
-    dev_free(ph->rec_packed);
-    dev_free(ph->rec_soa);
+    if (ph->arena) {
+        // walks of any stream may still gather from it, as hipFree would wait for them
+        if (hipDeviceSynchronize() == hipSuccess) ph->pool->put(ph->arena, ph->arena_bytes);
+        else dev_free(ph->arena);
+    }
     delete ph;
 }
 
@@ -599,8 +710,7 @@ SW_API int sw_phantom_generate(sw_engine *e, const uint64_t dims[3], const float
         void **p[5];
         ~Tables() { for (void **q : p) dev_free(*q); }
     } tables{{(void **)&dcyl, (void **)&dsph, (void **)&dstart, (void **)&daxn, (void **)&dastart}};
-    SW_HIP(e, hipMalloc((void **)&ph->mask, ph->n));
-    SW_HIP(e, hipMalloc((void **)&ph->field, ph->n * sizeof(float)));
+    if ((rc = phantom_alloc(e, ph.get(), formats))) return rc;
     SW_HIP(e, dev_upload(&dcyl, cyl.data(), cyl.size(), s));
     SW_HIP(e, dev_upload(&dsph, sorted.data(), sorted.size(), s));
     SW_HIP(e, dev_upload(&dstart, start.data(), start.size(), s));

@@ -100,12 +100,10 @@ SW_HD U32x4 philox4x32_10_pre(uint32_t c0, uint32_t c1, uint32_t m_hi, uint32_t 
 
 // philox4x32_10_pre for a counter (att, spin, 0) whose attempt word `att` and key
 // are uniform across the wave: round 1's first product and round 2's second are
-// then scalar, and the words they meet fold on the scalar unit.
+// then scalar, and the words they meet fold on the scalar unit.  The round keys are
+// left to the compiler, which keeps them in scalar registers across the step loop.
 SW_HD U32x4 philox4x32_10_uniform(uint64_t att, uint32_t m_hi, uint32_t m_lo, uint32_t k0, uint32_t k1) {
     constexpr uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
-#if defined(__HIP_DEVICE_COMPILE__) && 0
-    asm volatile("" : "+s"(k0), "+s"(k1));
-#endif
     uint32_t c0, c1, c2, c3;
     {
         const uint64_t p0 = (uint64_t)kPhiloxM0 * (uint32_t)att;          // round 1
