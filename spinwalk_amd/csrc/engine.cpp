@@ -1110,11 +1110,13 @@ struct sw_batch {
     unsigned long long *d_counters = nullptr;    // [n_items][4]
     sw::Excitation *d_exc = nullptr;             // every tile's excitation table
     uint32_t *d_order = nullptr;                 // every tile's visiting order
-    double *d_partial = nullptr;                 // echo-reduction scratch
+    // the tiles' echo sums: one launch per pass over d_reduce, with scratch of every tile
+    sw::ReduceItem *d_reduce = nullptr;
+    double *d_partial = nullptr;
+    uint32_t reduce_blocks = 0, reduce_pairs = 0;
     struct Group { int variant; int views; uint32_t offset, n_slots; };
     std::vector<Group> groups;
-    struct Reduce { const void *M1; int f64; const uint8_t *T; uint32_t n, n_te, n_sub; double *out; };
-    std::vector<Reduce> reduces;
+    std::vector<sw::ReduceItem> reduces;
     int rng = 0, field = 0, prec = 0;
     bool idx32 = false;
     bool mixed = false;                          // 64-bit mode over items in both packed layouts
@@ -1172,10 +1174,9 @@ hipError_t batch_enqueue(const sw_batch *b, hipStream_t s) {
                                     lds, s);
         if (err != hipSuccess) return err;
     }
-    for (const auto &r : b->reduces) {
-        err = sw::launch_echo_reduce(r.M1, r.f64, r.T, r.n, r.n_te, r.n_sub, b->d_partial, r.out, s);
-        if (err != hipSuccess) return err;
-    }
+    if (!b->reduces.empty())
+        return sw::launch_echo_reduce_batch(b->d_reduce, (uint32_t)b->reduces.size(), b->reduce_blocks,
+                                            b->reduce_pairs, s);
     return hipSuccess;
 }
 
@@ -1386,7 +1387,7 @@ void batch_free(sw_batch *b) {
         (void)hipEventDestroy(b->run_ev);
     }
     for (void *x : {(void *)b->d_items, (void *)b->d_fused, (void *)b->d_chunks, (void *)b->d_counters,
-                    (void *)b->d_exc, (void *)b->d_order, (void *)b->d_partial})
+                    (void *)b->d_exc, (void *)b->d_order, (void *)b->d_partial, (void *)b->d_reduce})
         dev_free(x);
     delete b;
 }
@@ -1435,12 +1436,16 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         order_off[i] = n_order;
         if (it.opts.spatial_order && it.opts.n_local > 1) n_order += it.opts.n_local;
         if (it.d_echo_sums) {
-            sw_batch::Reduce r;
+            sw::ReduceItem r{};
             r.M1 = it.d_M1; r.f64 = it.opts.precision == SW_PREC_F64; r.T = it.d_T;
             r.n = it.opts.n_local; r.n_te = it.sequence->n_te; r.n_sub = it.sequence->n_sub; r.out = it.d_echo_sums;
             if (r.n_te && r.n_sub) {
+                r.first_block = b->reduce_blocks;
+                r.first_pair = b->reduce_pairs;
+                b->reduce_blocks += sw::reduce_blocks(r.n, r.n_te, r.n_sub);
+                b->reduce_pairs += sw::reduce_pairs(r.n, r.n_te, r.n_sub);
                 b->reduces.push_back(r);
-                partial = std::max(partial, (size_t)sw::reduce_partial_len(r.n, r.n_te, r.n_sub));
+                partial += (size_t)sw::reduce_partial_len(r.n, r.n_te, r.n_sub);
             }
         }
     }
@@ -1451,7 +1456,15 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
     SW_HIP(e, hipMalloc((void **)&b->d_counters, 4 * n_items * sizeof(unsigned long long)));
     SW_HIP(e, dev_upload(&b->d_exc, exc.data(), exc.size(), s));
     if (n_order) SW_HIP(e, hipMalloc((void **)&b->d_order, n_order * sizeof(uint32_t)));
-    if (partial) SW_HIP(e, hipMalloc((void **)&b->d_partial, partial * sizeof(double)));
+    if (!b->reduces.empty()) {
+        SW_HIP(e, hipMalloc((void **)&b->d_partial, partial * sizeof(double)));
+        size_t off = 0;
+        for (auto &r : b->reduces) {
+            r.partial = b->d_partial + off;
+            off += (size_t)sw::reduce_partial_len(r.n, r.n_te, r.n_sub);
+        }
+        SW_HIP(e, dev_upload(&b->d_reduce, b->reduces.data(), b->reduces.size(), s));
+    }
     int rc0 = scratch_acquire(e, s);             // build_order_into uses the engine's sort scratch
     if (rc0) return rc0;
     for (uint32_t i = 0; i < n_items; i++) {
@@ -1791,8 +1804,10 @@ SW_API int sw_echo_reduce_device(sw_engine *e, const void *d_M1, int m1_dtype, c
         SW_HIP(e, hipMalloc((void **)&e->d_partial, need * sizeof(double)));
         e->partial_cap = need;
     }
-    SW_HIP(e, sw::launch_echo_reduce(d_M1, m1_dtype == SW_DTYPE_F64, d_T, n_spins, n_te, n_sub, e->d_partial, d_out,
-                                     s));
+    sw::ReduceItem r{};
+    r.M1 = d_M1; r.T = d_T; r.partial = e->d_partial; r.out = d_out;
+    r.n = n_spins; r.n_te = n_te; r.n_sub = n_sub; r.f64 = m1_dtype == SW_DTYPE_F64;
+    SW_HIP(e, sw::launch_echo_reduce(r, s));
     return scratch_release(e, s);
 }
 

@@ -66,12 +66,22 @@ hipError_t launch_records(const uint8_t *mask, const float *field, uint64_t nx, 
 // records (kSoaF32) single walks gather; `out` must be zero-filled for padding.
 hipError_t launch_f32_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz,
                               bool soa, void *out, hipStream_t s);
-// FP64 echo reduction into out[(te*n_sub+label)*3 + {0,1,2}]; partial is scratch
-// of reduce_partial_len(n_spins, n_te, n_sub) doubles.
+// FP64 echo reduction into out[(te*n_sub+label)*3 + {0,1,2}].  partial is scratch
+// of reduce_partial_len(n, n_te, n_sub) doubles.
+struct ReduceItem {
+    const void *M1;
+    const uint8_t *T;
+    double *partial, *out;
+    uint32_t n, n_te, n_sub, f64;
+    uint32_t first_block, first_pair;      // the item's first of a batch's launches
+};
 uint64_t reduce_partial_len(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);
-hipError_t launch_echo_reduce(const void *M1, int f64, const uint8_t *T, uint32_t n_spins,
-                              uint32_t n_te, uint32_t n_sub, double *partial, double *out,
-                              hipStream_t s);
+uint32_t reduce_blocks(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);
+uint32_t reduce_pairs(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);      // that need the second pass
+hipError_t launch_echo_reduce(const ReduceItem &r, hipStream_t s);
+// Every item of items[] (device memory; n_blocks and n_pairs in all), one launch per pass.
+hipError_t launch_echo_reduce_batch(const ReduceItem *items, uint32_t n_items, uint32_t n_blocks, uint32_t n_pairs,
+                                    hipStream_t s);
 
 // The fixed scratch of the no-allocation walk (noalloc.hip): its size, and the
 // device address of `device`'s copy, looked up once per device (`device` must
