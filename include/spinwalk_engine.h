@@ -108,7 +108,8 @@ typedef struct sw_walk_opts {
     int32_t  rng;              /* SW_RNG_*                                              */
     int32_t  precision;        /* SW_PREC_*; SW_PREC_F64 writes M1 as double          */
     int32_t  field_format;     /* which phantom copy to gather (SW_FIELD_*)            */
-    int32_t  spatial_order;    /* 1 = visit spins in start-voxel brick order           */
+    int32_t  spatial_order;    /* 1 = visit spins in start-voxel brick order where that is the faster way (results
+                                  are the same; single walks of few spins or small phantoms go unsorted) */
     const float *replay_normals;  uint64_t replay_normal_stride;   /* device, [n_local][stride] */
     const float *replay_uniforms; uint64_t replay_uniform_stride;  /* device, [n_local][stride] */
     int32_t  step_loop;        /* SW_STEP_LOOP_*; 0 (auto) when zero-initialised       */

@@ -996,6 +996,26 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
 
 }  // namespace
 
+namespace {
+
+// Whether a single walk that asks for spatial order gets it.  Sorted spins share
+// lines with their neighbours, which pays when more spins are in flight than the
+// L2s (8 of 4 MiB in 128-byte lines: 262144) hold lines for, each its own.  Below
+// that every spin keeps its line by itself, and order only costs: its launches, and
+// waves of neighbours, some of which all meet vessel walls and redraw while others
+// are long done.  The same when the records fit each L2.  Sorted time over unsorted
+// (800 steps, FP32): 256^3 1.20 at 6.5e4 spins, 1.18 at 1.3e5, 0.98 to 1.10 at 2e5, 0.74
+// to 0.94 at 3e5, 0.52 at 1e6; 600^3 1.14 at 1.3e5, 1.10 at 2.1e5; int16 records of
+// 200^3 1.22 at 1.3e5, 1.04 at 2.4e5, 0.84 at 3e5; 64^3, whose records fit, 1.35 at 1.3e5
+// and 1.25 at 5e5.  PGSE trains on packed axons 0.98 to 1.04 at 6e4 to 2.1e5.
+constexpr uint32_t kUnsortedSpins = 208u << 10;
+constexpr uint64_t kUnsortedBytes = 4ull << 20;
+bool order_pays(const sw::WalkArgs &a, int field, bool replay) {
+    return a.n_local > kUnsortedSpins && sw::walk_mode(a, field, replay ? 1 : 0).bytes >= kUnsortedBytes;
+}
+
+}  // namespace
+
 SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence *cq, const sw_params *p,
                           const sw_walk_opts *o, const float *d_M0, const float *d_XYZ0, void *d_M1,
                           float *d_XYZ1, uint8_t *d_T, void *stream, sw_walk_stats *stats) {
@@ -1014,7 +1034,7 @@ SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence 
     a.exc = q->exc;
     a.counters = e->d_counters;
     a.order = nullptr;
-    if (o->spatial_order && o->n_local > 1) {
+    if (o->spatial_order && order_pays(a, field, o->rng == SW_RNG_REPLAY)) {
         rc = build_order(e, a, s);
         if (rc) return rc;
         a.order = e->d_order;
@@ -1075,10 +1095,12 @@ SW_API int sw_walk_device_noalloc(sw_engine *e, const sw_phantom *ph, const sw_s
                                              std::to_string(256 + order_bytes + plan.total_bytes) +
                                              " bytes of scratch; the no-allocation scratch holds " +
                                              std::to_string(cap) + " (use spatial_order 0 or sw_walk_device)");
-        uint32_t *order = (uint32_t *)(base + 256);
-        SW_HIP(e, sw::launch_spatial_order(plan, base + 256 + order_bytes, a.XYZ0, a.xyz_scale, o->n_local, a.s2g,
-                                           a.nx, a.ny, a.nz, order, s));
-        a.order = order;
+        if (order_pays(a, field, o->rng == SW_RNG_REPLAY)) {
+            uint32_t *order = (uint32_t *)(base + 256);
+            SW_HIP(e, sw::launch_spatial_order(plan, base + 256 + order_bytes, a.XYZ0, a.xyz_scale, o->n_local, a.s2g,
+                                               a.nx, a.ny, a.nz, order, s));
+            a.order = order;
+        }
     }
     SW_HIP(e, sw::launch_zero_u64(a.counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
