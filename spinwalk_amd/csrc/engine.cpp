@@ -1014,6 +1014,36 @@ bool order_pays(const sw::WalkArgs &a, int field, bool replay) {
     return a.n_local > kUnsortedSpins && sw::walk_mode(a, field, replay ? 1 : 0).bytes >= kUnsortedBytes;
 }
 
+// Whether the waves on a SIMD are held to kCapWaves.  Each spin in flight comes
+// back to the line it last read; the waves that fit a SIMD (8) hold twice the lines
+// of an L2, kCapWaves half of one XCD's, so fewer waves wait less.  It pays when
+//  - the records the spins in flight meet exceed an L2 (kCapWindow): the whole
+//    phantom when unsorted, an eighth (an XCD's part) when sorted, and of it the
+//    share of its spins that 8 waves are;
+//  - there are 6 waves a SIMD or more, so that the last round is not a fraction of
+//    the others (4 and a bit waves would take two rounds for one).
+// Uncapped time over capped, single walks: FP32 records of 256^3
+// 1.26 at 4e5 spins, 1.15 at 5e5, 1.10 at 1e6, 1.03 at 1.5e6; 400^3 1.08; 128^3 (window
+// 1 MiB) 0.95 to 0.99, so not capped.  int16 records of 400^3 1.54 at 5e5, 1.37 at 8e5
+// (bSSFP), 1.13 at 1.5e6; of 256^3 1.18 at 4e5, 1.02 at 7e5, 0.99 at 8e5 (window 2.7).
+// 3e5 spins (4.6 waves) 0.82 to 0.88 on 256^3.  Batches: 32 scales of 256^3, 1e5 spins
+// each, 116.7 -> 95.7 ms; 200^3 int16 0.95 fused.  Fused walks, which hold 5 waves anyway
+// and do more per gather: 1000^3 with 2e6 spins 117.4 -> 109.0 ms, int16 400^3 (window
+// 8.4 MiB) 0.99, FP32 400^3 (17 MiB) 1.13.
+constexpr uint64_t kWaveSpins = 64 * 1024;               // a wave on each of the 1024 SIMDs
+constexpr double kCapWindow = 2.8 * (1 << 20), kCapWindowFused = 12. * (1 << 20);
+bool cap_pays(uint64_t rec_bytes, uint64_t n_tile, uint64_t n_all, bool sorted, bool fused) {
+    double window = (double)rec_bytes;
+    if (sorted) window *= std::min(1., 8. * (double)kWaveSpins / (double)n_tile) / 8;
+    return n_all >= 6 * kWaveSpins && window > (fused ? kCapWindowFused : kCapWindow);
+}
+
+// Trajectories and replayed draws stream from HBM and keep every wave they can.
+uint32_t single_cap(const sw::WalkArgs &a, int field, bool replay) {
+    return !replay && !a.record_traj &&
+           cap_pays(sw::walk_mode(a, field, 0).bytes, a.n_local, a.n_local, a.order != nullptr, false);
+}
+
 }  // namespace
 
 SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence *cq, const sw_params *p,
@@ -1039,6 +1069,7 @@ SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence 
         if (rc) return rc;
         a.order = e->d_order;
     }
+    a.cap = single_cap(a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(e->d_counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
     SW_HIP(e, sw::launch_walk(a, o->rng == SW_RNG_REPLAY ? 1 : 0, field, o->precision, s));
@@ -1102,6 +1133,7 @@ SW_API int sw_walk_device_noalloc(sw_engine *e, const sw_phantom *ph, const sw_s
             a.order = order;
         }
     }
+    a.cap = single_cap(a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(a.counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
     SW_HIP(e, sw::launch_walk(a, o->rng == SW_RNG_REPLAY ? 1 : 0, field, o->precision, s));
@@ -1558,7 +1590,19 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         SW_HIP(e, hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
         b->lds_block = (size_t)v;
     }
-    int rc = apply_schedule(e, b.get(), kDefaultSchedule, s, true);
+    // capped where that pays for the walks that make up more than half of the spin-steps
+    sw_batch_schedule sched = kDefaultSchedule;
+    uint64_t n_all = 0, all = 0, capped = 0;
+    for (const auto &t : b->tiles) n_all += t.n_local;
+    for (const auto &t : b->tiles) {
+        const sw::WalkArgs &x = t.views == 1 ? singles[t.index] : fused[t.index].a;
+        const uint64_t bytes = sw::walk_mode(x, b->field, b->rng == SW_RNG_REPLAY ? 1 : 0).bytes;
+        all += t.cost * t.n_local;
+        if (!x.record_traj && cap_pays(bytes, t.n_local, n_all, x.order != nullptr, t.views > 1))
+            capped += t.cost * t.n_local;
+    }
+    if (b->rng != SW_RNG_REPLAY && 2 * capped > all) sched.waves_per_simd = sw::kCapWaves;
+    int rc = apply_schedule(e, b.get(), sched, s, true);
     if (rc) return rc;
     *out = b.release();
     return SW_OK;

@@ -1609,16 +1609,16 @@ template <class Rng, class F, class P, bool PAIRS>
 hipError_t launch_fp_loop(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
     const WalkMode m = mode_of<F>(a);
     const bool idx32 = m.idx32;
-    const size_t lds = m.lds;
+    const size_t lds = capped_lds(a, idx32 ? m.lds : 0);
     if constexpr (F::kPacked) {
         if (!idx32 && a.super_blocks) return hipErrorInvalidValue;   // super-blocks always fit the 32-bit mode
     }
     if (a.cross_fov) {
         if (idx32) hipLaunchKernelGGL((walk_kernel<Rng, F, P, true, true, PAIRS>), grid, block, lds, s, a);
-        else       hipLaunchKernelGGL((walk_kernel<Rng, F, P, true, false, PAIRS>), grid, block, 0, s, a);
+        else       hipLaunchKernelGGL((walk_kernel<Rng, F, P, true, false, PAIRS>), grid, block, lds, s, a);
     } else {
         if (idx32) hipLaunchKernelGGL((walk_kernel<Rng, F, P, false, true, PAIRS>), grid, block, lds, s, a);
-        else       hipLaunchKernelGGL((walk_kernel<Rng, F, P, false, false, PAIRS>), grid, block, 0, s, a);
+        else       hipLaunchKernelGGL((walk_kernel<Rng, F, P, false, false, PAIRS>), grid, block, lds, s, a);
     }
     return hipGetLastError();
 }
@@ -1629,8 +1629,9 @@ hipError_t launch_prod(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) 
     if constexpr (F::kPacked) {
         if (!m.idx32 && a.super_blocks) return hipErrorInvalidValue;   // super-blocks always fit the 32-bit mode
     }
-    if (m.idx32) hipLaunchKernelGGL((walk_prod_kernel<F, P, true, ONE_TR, TRAJ>), grid, block, m.lds, s, a);
-    else         hipLaunchKernelGGL((walk_prod_kernel<F, P, false, ONE_TR, TRAJ>), grid, block, 0, s, a);
+    const size_t lds = capped_lds(a, m.idx32 ? m.lds : 0);
+    if (m.idx32) hipLaunchKernelGGL((walk_prod_kernel<F, P, true, ONE_TR, TRAJ>), grid, block, lds, s, a);
+    else         hipLaunchKernelGGL((walk_prod_kernel<F, P, false, ONE_TR, TRAJ>), grid, block, lds, s, a);
     return hipGetLastError();
 }
 
