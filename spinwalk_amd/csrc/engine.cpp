@@ -876,6 +876,17 @@ int build_order(sw_engine *e, const sw::WalkArgs &a, hipStream_t s) {
     return build_order_into(e, a, e->d_order, s);
 }
 
+// Spins per wave of a single walk.  A wave takes as long as the slowest of its lanes,
+// the one that meets the most vessel walls and redraws, and a SIMD with one wave waits
+// out every latency of it.  So where waves of half as many spins still find a SIMD
+// each, half the lanes stay empty, 64 lanes against 32: 64^3, GRE of 400 steps, 1e3
+// spins 260 -> 238 us, 3.2e4 302 -> 275; 256^3, 3e2 spins 182 -> 184 us, 2e3 219 -> 214,
+// 3.2e4 288 -> 263; bSSFP of 20 dummies 1.38 -> 1.25 ms at 8e3; replayed spin echo of
+// 2e4 spins 1.26 -> 0.93 ms.  Shorter waves lose again below 2 blocks a CU (8 lanes: 0.6 to
+// 0.75 of the rate of 64 at 1e3 spins), and above the line the waves share issue slots
+// (32 lanes 1.00 of the rate at 6.5e4 spins, 0.86 at 1e5).
+uint32_t single_lanes(uint32_t n_local) { return n_local <= 32u * 1024 ? 32 : 64; }
+
 // Checks one walk's arguments and fills its WalkArgs, except exc, order and
 // counters.  *field_out receives the record format the walk gathers.
 int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, const sw_params *p,
@@ -986,6 +997,7 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
     // results).  Replayed walks and batches take one attempt per trip.
     if (o->step_loop < SW_STEP_LOOP_AUTO || o->step_loop > SW_STEP_LOOP_TWO)
         return fail(e, SW_E_INVALID, "unknown step_loop");
+    a.lanes = single_lanes(a.n_local);
     a.pairs = 0;
     if (o->rng == SW_RNG_PHILOX) {
         if (o->step_loop == SW_STEP_LOOP_TWO) a.pairs = 1;

@@ -157,6 +157,7 @@ struct WalkArgs {
     float           nf[3];        // nx, ny, nz as floats: the FoV in voxels
     double          vs[3];        // fov / n in double (the FP64 walk's gradient phase)
     float           g2d;          // (float) 1e-3 dt 1e-6 gamma rad2deg: mT/m x m -> degrees
+    uint32_t        lanes;        // a single walk's spins per wave (single_lanes)
 
     // ---- sequence tables (device) -------------------------------------------
     const double   *diffusivity;  // [n_sub] metres per axis per step

@@ -951,12 +951,11 @@ done:
     return st;
 }
 
-// One workgroup walks the spins at positions [t0, t0 + spl * blockDim.x) of the
-// launch's visiting order (fewer at the end): lane l takes positions
-// t0 + k * blockDim.x + l, k = 0 .. spl-1, one after the other.
 template <class Rec, class Phase, bool CROSS, bool IDX32, int NV>
 __device__ int walk_spin_pairs(const WalkArgs &a, const WalkView *xv, uint32_t li, uint64_t &n_acc, uint32_t &n_rej);
 
+// This lane walks the spins at positions t0 + k * blockDim.x, k = 0 .. spl-1, of
+// the launch's visiting order, those below n_local, one after the other.
 // PAIRS: the production step loop with two attempts per trip (walk_spin_pairs).
 template <class Rng, class Rec, class Phase, bool CROSS, bool IDX32, bool PAIRS = false>
 __device__ __forceinline__ void walk_block(const WalkArgs &a, uint32_t t0, uint32_t spl = 1) {
@@ -969,7 +968,7 @@ __device__ __forceinline__ void walk_block(const WalkArgs &a, uint32_t t0, uint3
     uint64_t n_acc = 0;
     uint32_t n_rej = 0, lost = 0, exh = 0;
     for (uint32_t k = 0; k < spl; k++) {
-        const uint32_t t = t0 + k * blockDim.x + threadIdx.x;
+        const uint32_t t = t0 + k * blockDim.x;
         if (t < a.n_local) {
             const uint32_t li = a.order ? a.order[t] : t;
             int st;
@@ -1516,6 +1515,13 @@ __device__ __forceinline__ void walk_block_views(const WalkArgs &a, const WalkVi
 // The two-attempt loop holds a second position, record and two draw bundles
 // more: it is compiled for 4 waves per SIMD (up to 128 registers), which it
 // keeps busy with two gathers in flight per wave.
+// The position in the visiting order of this lane of a single walk's block: waves of
+// 64 spins, or of the first `lanes` lanes with a spin each.
+__device__ __forceinline__ uint32_t single_position(uint32_t lanes, uint32_t block) {
+    const uint32_t lane = threadIdx.x & 63;
+    return lane < lanes ? (block * (blockDim.x >> 6) + (threadIdx.x >> 6)) * lanes + lane : ~0u;
+}
+
 template <class Rng, class Rec, class Phase, bool CROSS, bool IDX32, bool PAIRS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIRS ? SW_PAIR_WAVES_PER_EU : SW_WALK_WAVES_PER_EU)))
 void walk_kernel(const WalkArgs a) {
@@ -1524,7 +1530,7 @@ void walk_kernel(const WalkArgs a) {
     // The grid is a multiple of 8 blocks, so the remap is a permutation.
     const uint32_t per = gridDim.x / 8, b = blockIdx.x;
     const uint32_t lb = (b % 8) * per + b / 8;
-    walk_block<Rng, Rec, Phase, CROSS, IDX32, PAIRS>(a, lb * blockDim.x);
+    walk_block<Rng, Rec, Phase, CROSS, IDX32, PAIRS>(a, single_position(a.lanes, lb));
 }
 
 // The production walk with one attempt per trip (walk_prod.hpp).  The arguments
@@ -1534,7 +1540,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SW_WALK_WAV
 void walk_prod_kernel(const WalkArgs) {
     const uint32_t per = gridDim.x / 8, b = blockIdx.x;
     const uint32_t lb = (b % 8) * per + b / 8;
-    prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>((ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), nullptr, 1, lb * blockDim.x, 1);
+    const ArgsPtr a = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>(a, nullptr, 1, single_position(a->lanes, lb), 1);
 }
 
 // The batched walk: block b takes the chunk at slot (b mod 8) * (grid / 8) + b / 8
@@ -1563,7 +1570,7 @@ void walk_batch_kernel(const void *__restrict__ items, const BatchChunk *__restr
     const BatchChunk c = chunks[(b % 8) * per + b / 8];
     if (c.item == kNoItem) return;                    // padding slot (uniform across the block)
     if constexpr (NV == 1) {
-        walk_block<Rng, Rec, Phase, CROSS, IDX32>(((const WalkArgs *)items)[c.item], c.first, spl);
+        walk_block<Rng, Rec, Phase, CROSS, IDX32>(((const WalkArgs *)items)[c.item], c.first + threadIdx.x, spl);
     } else {
         const FusedArgs &f = ((const FusedArgs *)items)[c.item];
         walk_block_views<Rng, Rec, Phase, CROSS, IDX32, NV>(f.a, f.xv, f.n_views, c.first, spl);
@@ -1578,10 +1585,11 @@ void walk_batch_prod_kernel(const void *__restrict__ items, const BatchChunk *__
     const BatchChunk c = chunks[(b % 8) * per + b / 8];
     if (c.item == kNoItem) return;                    // padding slot (uniform across the block)
     if constexpr (NV == 1) {
-        prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>((ArgsPtr)((const WalkArgs *)items + c.item), nullptr, 1, c.first, spl);
+        prod_block<Rec, Phase, IDX32, 1, ONE_TR, TRAJ>((ArgsPtr)((const WalkArgs *)items + c.item), nullptr, 1,
+                                                       c.first + threadIdx.x, spl);
     } else {
         const auto *f = (const __attribute__((address_space(4))) FusedArgs *)((const FusedArgs *)items + c.item);
-        prod_block<Rec, Phase, IDX32, NV, ONE_TR, TRAJ>(&f->a, f->xv, f->n_views, c.first, spl);
+        prod_block<Rec, Phase, IDX32, NV, ONE_TR, TRAJ>(&f->a, f->xv, f->n_views, c.first + threadIdx.x, spl);
     }
 }
 
@@ -1723,7 +1731,7 @@ hipError_t launch_batch_half(const void *items, const BatchChunk *chunks, uint32
 
 template <class Rng, class P>
 hipError_t launch_wide(const WalkArgs &a, int field, hipStream_t s) {
-    const uint32_t nb = (a.n_local + 255) / 256;
+    const uint32_t nb = (a.n_local + 4 * a.lanes - 1) / (4 * a.lanes);
     if (nb == 0) return hipSuccess;
     const dim3 block(256), grid((nb + 7) / 8 * 8);
     if (field == 0) return launch_fp<Rng, RecNone, P>(a, s, grid, block);
@@ -1732,7 +1740,7 @@ hipError_t launch_wide(const WalkArgs &a, int field, hipStream_t s) {
 }
 template <class Rng, class P>
 hipError_t launch_half(const WalkArgs &a, int field, hipStream_t s) {
-    const uint32_t nb = (a.n_local + 255) / 256;
+    const uint32_t nb = (a.n_local + 4 * a.lanes - 1) / (4 * a.lanes);
     if (nb == 0) return hipSuccess;
     const dim3 block(256), grid((nb + 7) / 8 * 8);
     if (field == 2) return launch_fp<Rng, RecF16, P>(a, s, grid, block);

@@ -401,9 +401,8 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
     return st;
 }
 
-// One workgroup walks the spins at positions [t0, t0 + spl * blockDim.x) of the
-// launch's visiting order (fewer at the end): lane l takes positions
-// t0 + k * blockDim.x + l, k = 0 .. spl-1, one after the other.
+// This lane walks the spins at positions t0 + k * blockDim.x, k = 0 .. spl-1, of
+// the launch's visiting order, those below n_local, one after the other.
 template <class Rec, class Phase, bool IDX32, int NV, bool ONE_TR, bool TRAJ>
 __device__ __forceinline__ void prod_block(ArgsPtr a, ViewPtr xv, uint32_t n_views, uint32_t t0, uint32_t spl) {
     if (IDX32) {
@@ -415,7 +414,7 @@ __device__ __forceinline__ void prod_block(ArgsPtr a, ViewPtr xv, uint32_t n_vie
     uint64_t n_acc = 0;
     uint32_t n_rej = 0, lost = 0;
     for (uint32_t k = 0; k < spl; k++) {
-        const uint32_t t = t0 + k * blockDim.x + threadIdx.x;
+        const uint32_t t = t0 + k * blockDim.x;
         if (t < a->n_local)
             lost += walk_spin_prod<Rec, Phase, IDX32, NV, ONE_TR, TRAJ>(a, xv, a->order ? a->order[t] : t, n_acc, n_rej) == ST_LOST;
     }
