@@ -530,23 +530,12 @@ static int phantom_finish(sw_engine *e, sw_phantom *ph, uint32_t formats) {
     for (int f = 0; f <= SW_FIELD_Q16; f++) {
         const bool want = (f == SW_FIELD_NONE) ? !ph->has_field : (ph->has_field && (formats & (1u << f)));
         if (!want) continue;
-        if (f == SW_FIELD_F32 || f == SW_FIELD_NONE) {
-            const sw::BrickShape sh = f == SW_FIELD_F32 ? sw::kBrick8 : sw::kBrick4;
-            SW_HIP(e, hipMemsetAsync(ph->rec[f], 0, ((size_t)(sw::brick_count(nx, sh.lbx) * sw::brick_count(ny, sh.lby) *
-                                     sw::brick_count(nz, sh.lbz)) << (sh.lbx + sh.lby + sh.lbz)) * (f == SW_FIELD_F32 ? 8 : 4), s));
-        } else {
-            SW_HIP(e, hipMemsetAsync(ph->rec[f], 0, (size_t)sw::pack_bytes(nx, ny, nz, sw::kPack16, sw::pack_super(nx, ny, nz, sw::kPack16)), s));
-        }
         const int kind = f == SW_FIELD_F32 ? 0 : f == SW_FIELD_F16 ? 1 : f == SW_FIELD_BF16 ? 2 : f == SW_FIELD_Q16 ? 4 : 3;
         SW_HIP(e, sw::launch_records(ph->mask, ph->field, nx, ny, nz, kind,
                                      1.0f / (f == SW_FIELD_Q16 ? ph->q_scale : ph->half_scale), ph->rec[f], s));
         if (f == SW_FIELD_F32) {         // the production walks' copies: packed for batches, SoA for single walks
-            const size_t bytes = (size_t)sw::pack_bytes(nx, ny, nz, sw::kPackF32, sw::pack_super(nx, ny, nz, sw::kPackF32));
-            for (int soa = 0; soa < 2; soa++) {
-                void *r = soa ? ph->rec_soa : ph->rec_packed;
-                SW_HIP(e, hipMemsetAsync(r, 0, bytes, s));
-                SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, soa != 0, r, s));
-            }
+            SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, false, ph->rec_packed, s));
+            SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, true, ph->rec_soa, s));
         }
     }
     SW_HIP(e, hipStreamSynchronize(s));

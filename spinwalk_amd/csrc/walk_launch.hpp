@@ -64,12 +64,12 @@ hipError_t launch_phantom_stats(const uint8_t *mask, const float *field, uint64_
 // Row-major mask/field -> bricked voxel records: kind 0 Rec8 f32, 3 Rec4 label
 // only; kinds 1 fp16, 2 bf16 and 4 int16 fixed point as packed 3-byte records
 // (kPack16).  inv_scale divides the field before the 16-bit kinds round it.
-// `out` must be zero-filled for padding.
+// Every line of `out` is written, padding included.
 hipError_t launch_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz, int kind,
                           float inv_scale, void *out, hipStream_t s);
 // Row-major mask/field -> the float32 bricks of production walks: the packed
 // 5-byte records (kPackF32) batches gather, or with soa the structure-of-arrays
-// records (kSoaF32) single walks gather; `out` must be zero-filled for padding.
+// records (kSoaF32) single walks gather; every line of `out` is written, padding included.
 hipError_t launch_f32_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz,
                               bool soa, void *out, hipStream_t s);
 // FP64 echo reduction into out[(te*n_sub+label)*3 + {0,1,2}].  partial is scratch
