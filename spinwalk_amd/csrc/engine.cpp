@@ -992,6 +992,9 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
         if (o->step_loop == SW_STEP_LOOP_TWO) a.pairs = 1;
         else if (o->step_loop == SW_STEP_LOOP_AUTO) a.pairs = sw::walk_mode(a, field, 0).bytes > kPairsMinBytes ? 1u : 0u;
     }
+    // staging columns where the workgroup's 64 KiB of LDS hold them with the tables
+    a.stage = sw::stage_wanted(a, o->rng == SW_RNG_REPLAY) && !a.pairs &&
+              sw::walk_mode(a, field, o->rng == SW_RNG_REPLAY ? 1 : 0).lds + sw::stage_lds(256) <= 65536 ? 1u : 0u;
     return SW_OK;
 }
 
@@ -1174,6 +1177,7 @@ struct sw_batch {
     std::vector<sw::ReduceItem> reduces;
     int rng = 0, field = 0, prec = 0;
     bool idx32 = false;
+    bool stage = false;                          // and staging columns (WalkArgs::stage)
     bool mixed = false;                          // 64-bit mode over items in both packed layouts
     size_t lds = 0;                              // LDS of a workgroup: per-axis tables, then tissue tables (32-bit mode)
     // what the chunk table is built from: per walk unit (a single tile, or a
@@ -1208,7 +1212,7 @@ namespace {
 // k = 256 * waves_per_simd / chunk_spins workgroups per CU; k fit when
 // k * L <= LDS per CU < (k + 1) * L, so L = LDS per CU / (k + 1/2).
 size_t batch_lds(const sw_batch &b, const sw_batch_schedule &sc) {
-    size_t lds = b.idx32 ? b.lds : 0;
+    size_t lds = (b.idx32 ? b.lds : 0) + (b.stage ? sw::stage_lds(sc.chunk_spins) : 0);
     if (sc.waves_per_simd && b.lds_cu && sc.chunk_spins) {
         const size_t k = (size_t)256 * sc.waves_per_simd / sc.chunk_spins;
         const size_t l = (size_t)(2 * b.lds_cu / (2 * k + 1)) & ~(size_t)1023;
@@ -1505,6 +1509,11 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         }
     }
     if (!b->idx32) b->lds = 0;
+    // Tiles stage where the largest tile's tables leave the room.
+    for (uint32_t i = 0; i < n_items; i++) {
+        args[i].stage = sw::stage_wanted(args[i], b->rng == SW_RNG_REPLAY) && b->lds + sw::stage_lds(256) <= 65536;
+        b->stage = b->stage || args[i].stage;
+    }
     for (uint32_t i = 0; i < n_items && !b->idx32; i++) b->mixed = b->mixed || args[i].super_blocks;
 
     // ---- device tables

@@ -175,6 +175,7 @@ struct WalkArgs {
     const int32_t  *TE_t;         uint32_t n_te;
     const int32_t  *deph_t;       const float *deph_deg; uint32_t n_deph;
     const int32_t  *grad_t;       const float *gx, *gy, *gz; uint32_t n_grad;
+    uint32_t        stage;        // 1: the workgroup has kStageBytes of LDS a lane after its tables (stage_column)
     const Excitation *exc;        // [n_dummy + 1]
     float           exc_s, exc_c; // param.s, param.c
     double          exc_sd, exc_cd;
@@ -211,6 +212,13 @@ constexpr uint32_t kTissueLdsMax = 16;
 SW_HD_INLINE uint32_t tissue_lds_words(const WalkArgs &a) {
     return a.tissue_lds ? a.n_sub * a.n_sub + 5 * a.n_sub : 0u;
 }
+
+// Staging in LDS, after a workgroup's tables: a ring of two 64-byte sectors of
+// recorded positions per lane.  Taken where it fits the 64 KiB of a workgroup and
+// kStageSpins rows or more are open (Recorder).
+constexpr uint32_t kStageBytes = 128, kStageSpins = 72u << 10;
+constexpr size_t stage_lds(uint32_t threads) { return (size_t)threads * kStageBytes + 16; }
+SW_HD_INLINE bool stage_wanted(const WalkArgs &a, bool replay) { return !replay && a.record_traj && a.n_local >= kStageSpins; }
 
 // The kernel a walk takes.  Production walks of a scan with one TR, and those that
 // record trajectories, take the step loop of walk_prod.hpp; scans with dummy TRs

@@ -273,6 +273,10 @@ __device__ __forceinline__ void after_draws(uint2 &r, float x, float y, float z)
     asm volatile("" : "+v"(r.x), "+v"(r.y) : "v"(x), "v"(y), "v"(z));
 }
 
+// A workgroup's dynamic LDS: the per-axis tables of the 32-bit mode, the tissue
+// tables, the staging columns.
+extern __shared__ __attribute__((aligned(16))) uint32_t axis_tab[];
+
 // ---------------------------------------------------------------------------
 // Draw sources.
 // ---------------------------------------------------------------------------
@@ -280,6 +284,12 @@ __device__ __forceinline__ void after_draws(uint2 &r, float x, float y, float z)
 // attempt available ahead of time (so they can be computed while the current
 // attempt's gathers are in flight); commit() consumes them.  An attempt that does
 // not move (diffusivity 0) consumes nothing, as in the reference (kernels.cu:130).
+// This wave's part of the staging rings in axis_tab, 16-byte aligned after the tables.
+template <bool IDX32, class A> __device__ __forceinline__ uint32_t stage_ring(const A &a) {
+    const uint32_t tables = IDX32 ? (uint32_t)(a.nx + a.ny + a.nz) + (a.tissue_lds ? a.n_sub * a.n_sub + 5 * a.n_sub : 0u) : 0u;
+    return ((tables + 3) & ~3u) + (threadIdx.x >> 6) * (64 * kStageBytes / 4);
+}
+
 struct ReplayRng {          // the reference CPU path's recorded streams
     static constexpr bool kReplay = true;
     const float *n, *u;
@@ -359,7 +369,6 @@ template <bool IDX32> struct Vox {
 // (b = subscript >> lb, L = lbx + lby + lbz; the parts occupy disjoint bits, so
 // the OR is a sum).  In the 32-bit mode each block keeps the three tables in LDS:
 // axis_tab[0, nx) = X, [nx, nx+ny) = Y, [nx+ny, nx+ny+nz) = Z.
-extern __shared__ uint32_t axis_tab[];
 
 // For the packed bricks the index is the record's byte offset, separable in the
 // same way (w bytes a record, brick coordinates b = i / brick side, super-blocks
@@ -1536,7 +1545,7 @@ void walk_kernel(const WalkArgs a) {
 // The production walk with one attempt per trip (walk_prod.hpp).  The arguments
 // are read where they are passed, in the constant address space.
 template <class Rec, class Phase, bool IDX32, bool ONE_TR, bool TRAJ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SW_WALK_WAVES_PER_EU)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TRAJ ? 4 : SW_WALK_WAVES_PER_EU)))
 void walk_prod_kernel(const WalkArgs) {
     const uint32_t per = gridDim.x / 8, b = blockIdx.x;
     const uint32_t lb = (b % 8) * per + b / 8;
@@ -1579,7 +1588,7 @@ void walk_batch_kernel(const void *__restrict__ items, const BatchChunk *__restr
 
 // The production form of walk_batch_kernel.
 template <class Rec, class Phase, bool IDX32, int NV, bool ONE_TR, bool TRAJ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(walk_waves_per_eu<Phase, NV>())))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TRAJ ? 4 : walk_waves_per_eu<Phase, NV>())))
 void walk_batch_prod_kernel(const void *__restrict__ items, const BatchChunk *__restrict__ chunks, uint32_t spl) {
     const uint32_t per = gridDim.x / 8, b = blockIdx.x;
     const BatchChunk c = chunks[(b % 8) * per + b / 8];
@@ -1637,7 +1646,7 @@ hipError_t launch_prod(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) 
     if constexpr (F::kPacked) {
         if (!m.idx32 && a.super_blocks) return hipErrorInvalidValue;   // super-blocks always fit the 32-bit mode
     }
-    const size_t lds = capped_lds(a, m.idx32 ? m.lds : 0);
+    const size_t lds = capped_lds(a, (m.idx32 ? m.lds : 0) + (a.stage ? stage_lds(block.x) : 0));
     if (m.idx32) hipLaunchKernelGGL((walk_prod_kernel<F, P, true, ONE_TR, TRAJ>), grid, block, lds, s, a);
     else         hipLaunchKernelGGL((walk_prod_kernel<F, P, false, ONE_TR, TRAJ>), grid, block, lds, s, a);
     return hipGetLastError();

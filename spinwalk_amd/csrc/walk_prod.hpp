@@ -239,6 +239,97 @@ __device__ __forceinline__ bool prod_outside(ArgsPtr a, const Hot &h, const floa
     return ok;
 }
 
+// Recorded positions on their way to XYZ1.  Each spin has a row of its own, so a
+// store per step is 64 pieces of 12 bytes in 64 lines, and the L2 sends nearly each of
+// them on by itself: 63 M write requests, 3.3 GB, for the 0.96 GB of 1e5 spins and 800
+// steps, which is what such walks wait for.  So a lane keeps its words in a ring of two
+// 64-byte sectors in LDS, and when some lane's ring is full the wave writes the whole
+// sectors: four lanes exchange pieces, so that each store of the four is one lane's
+// sector, aligned.  The ends of a row go word by word.  200^3: 1e5 spins of 800 steps 1.41
+// -> 0.85 ms, 2e5 of 400 1.99 -> 0.85 ms, 5e5 of 200 1.96 -> 0.96 ms.  Only from
+// kStageSpins on: with fewer rows open the L2 gathers the pieces itself, and the ring
+// costs more than it saves (5e4 spins 0.65 ms without, 0.74 with; 6.5e4 0.75 and 0.75;
+// 8e4 1.21 and 0.82).  Compiled for 4 waves a SIMD, which is what the rings leave room for
+// and where nothing of the step loop spills.
+// A lane's words: absolute word w (row words from the row's 64-byte boundary) in
+// piece w / 4 mod 8, the pieces 64 lanes apart.  Without room in LDS
+// (WalkArgs::stage) every step is written as it comes.
+typedef uint32_t Piece __attribute__((ext_vector_type(4)));
+typedef uint32_t PieceOut __attribute__((ext_vector_type(4), aligned(4)));
+template <bool IDX32> struct Recorder {
+    bool on;                     // staged
+    uint32_t ring;               // this lane's place in the wave's ring, axis_tab[ring ..]
+    uint32_t first, w, done;     // words: the row's first, the next, the first not yet written
+    float vs[3];
+    __device__ Recorder(ArgsPtr a, ViewPtr, uint64_t xoff)
+        : on(a->stage), ring(stage_ring<IDX32>(*a) + 4 * (threadIdx.x & 63)), vs{a->vsf[0], a->vsf[1], a->vsf[2]} {
+        first = w = done = (uint32_t)((uintptr_t)(a->XYZ1 + xoff) / 4) & (on ? 15u : 0u);
+    }
+    __device__ bool any() const { return w != first; }
+    // word i's place
+    __device__ uint32_t place(uint32_t i) const { return ring + (i & 28u) * 64 + (i & 3u); }
+    template <int NV> __device__ void add(ArgsPtr a, ViewPtr xv, uint64_t xoff, const float y[3]) {
+        if (!on) {
+            #pragma unroll
+            for (int v = 0; v < NV; v++) {
+                float *dst = SW_VIEW(a, xv, v, XYZ1) + xoff + w;
+                for (int i = 0; i < 3; i++) dst[i] = y[i] * vs[i];
+            }
+        } else {
+            for (uint32_t i = 0; i < 3; i++) axis_tab[place(w + i)] = __float_as_uint(y[i] * vs[i]);
+        }
+        w += 3;
+    }
+    // Called by every lane of the wave that still walks.
+    template <int NV> __device__ void spill(ArgsPtr a, ViewPtr xv, uint64_t xoff) {
+        if (on && __builtin_amdgcn_ballot_w64(w - (done & ~15u) > 29) != 0) write<NV>(a, xv, xoff);
+    }
+    template <int NV> __device__ void write(ArgsPtr a, ViewPtr xv, uint64_t xoff) {
+        // a row's first words, up to its first 64-byte boundary
+        if (done & 15u && w >= 16) words<NV>(a, xv, xoff, 16);
+        const bool full = w - done >= 16 && !(done & 15u);
+        __builtin_amdgcn_wave_barrier();                              // other lanes read what this one wrote
+        const uint64_t m = __builtin_amdgcn_ballot_w64(true);
+        const uint64_t q = m & m >> 1 & m >> 2 & m >> 3 & 0x1111111111111111ull;
+        const uint64_t off = xoff + done - first;                     // of the sector in XYZ1
+        if (q * 15 == m) {                                            // whole quads of lanes
+            const uint32_t st = full ? (done & 16u) | 1u : 0u;
+            exchange<0, NV>(a, xv, off, st);
+            exchange<1, NV>(a, xv, off, st);
+            exchange<2, NV>(a, xv, off, st);
+            exchange<3, NV>(a, xv, off, st);
+        } else if (full) {
+            #pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                const Piece p = *(const Piece *)(axis_tab + ring + ((done & 16u) + 4 * j) * 64);
+                #pragma unroll
+                for (int v = 0; v < NV; v++) *(PieceOut *)(SW_VIEW(a, xv, v, XYZ1) + off + 4 * j) = p;
+            }
+        }
+        if (full) done += 16;
+    }
+    // The sector of the quad's lane K: its lanes store a piece each.
+    template <int K, int NV> __device__ void exchange(ArgsPtr a, ViewPtr xv, uint64_t off, uint32_t st) {
+        const auto of_k = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, K * 0x55, 0xF, 0xF, true); };
+        const uint64_t o = (uint64_t)of_k((uint32_t)(off >> 32)) << 32 | of_k((uint32_t)off);
+        const uint32_t j4 = 4 * (threadIdx.x & 3);
+        st = of_k(st);
+        if (st) {
+            const Piece p = *(const Piece *)(axis_tab + ring + ((st & 16u) + j4) * 64 + 4 * K - j4);
+            #pragma unroll
+            for (int v = 0; v < NV; v++) *(PieceOut *)(SW_VIEW(a, xv, v, XYZ1) + o + j4) = p;
+        }
+    }
+    // this lane's words up to `end`, one by one
+    template <int NV> __device__ void words(ArgsPtr a, ViewPtr xv, uint64_t xoff, uint32_t end) {
+        for (; done < end; done++) {
+            const float f = __uint_as_float(axis_tab[place(done)]);
+            #pragma unroll
+            for (int v = 0; v < NV; v++) (SW_VIEW(a, xv, v, XYZ1) + xoff)[done - first] = f;
+        }
+    }
+};
+
 // One spin.  ONE_TR: the scan has no dummy TRs, so every lane of the wave that
 // still walks is at the same attempt, and the attempt counter and the draw's
 // first products run on the scalar unit.
@@ -258,10 +349,6 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
         x[i] = PosVox::start(*a, x0, i);
         #pragma unroll
         for (int v = 0; v < NV; v++) m[v][i] = (R)a->M0[3 * (uint64_t)li + i];
-        if (TRAJ) {
-            #pragma unroll
-            for (int v = 0; v < NV; v++) (SW_VIEW(a, xv, v, XYZ1) + xoff)[i] = x0;
-        }
     }
     Hot h;
     h.n[0] = (uint32_t)a->nx; h.n[1] = (uint32_t)a->ny; h.n[2] = (uint32_t)a->nz;
@@ -271,6 +358,7 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
     // HOT_TISSUE_LDS, HOT_CLOSED, HOT_CROSS of arguments that are 0 or 1
     h.flags = (IDX32 ? a->tissue_lds : 0u) | a->closed << 1 | (uint32_t)a->cross_fov << 2;
     int st = ST_OK;
+    bool recorded = false;
     uint32_t d = 0, tp = 0;
     const Vox<IDX32> vx = PosVox::find<Rec, IDX32>(*a, x);             // kernels.cu:102
     if (!vx.ok) {                                                      // the reference reads out of bounds here
@@ -279,7 +367,7 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
         typename Rec::T raw = rec_load<Rec, IDX32>(a->rec, vx.rec);
         uint32_t ts = Rec::label(raw);                                 // :103
         float step[3];
-        uint64_t slot = 0;
+        [[maybe_unused]] Recorder<IDX32> rec1(a, xv, xoff);
         uint64_t att = 0;
         uint32_t itr = 0, last_rej = 0;
         ProdDraw q = prod_draw<ONE_TR>(0, m_hi, m_lo, k0, k1);
@@ -363,18 +451,11 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
                     for (int v = 0; v < NV; v++) ph[v].add(f);         // :171
                     if (__builtin_expect(tp == ev.next, 0))
                         prod_events<Phase, NV>(cold(a), xv, ev, tp, ts, li, y, m, ph);
-                    if (TRAJ) {                                        // :218-221
-                        const ArgsPtr c = cold(a);
-                        #pragma unroll
-                        for (int v = 0; v < NV; v++) {
-                            float *dst = SW_VIEW(c, xv, v, XYZ1) + xoff + 3 * slot;
-                            for (int i = 0; i < 3; i++) dst[i] = PosVox::metres(*c, y[i], i);
-                        }
-                        ++slot;
-                    }
+                    if constexpr (TRAJ) rec1.template add<NV>(a, xv, xoff, y);   // :218-221
                     ++tp;
                 }
                 x[0] = y[0]; x[1] = y[1]; x[2] = y[2];
+                if constexpr (TRAJ) rec1.template spill<NV>(a, xv, xoff);
             }
             if (tp & kParked) { st = ST_LOST; tp &= ~kParked; break; }
             {
@@ -387,15 +468,22 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
             }
             if (last) { ++d; tp = 0; break; }                          // every TR done
         }
+        if constexpr (TRAJ) {
+            if (rec1.on) rec1.template words<NV>(a, xv, xoff, rec1.w);   // the row's last words, also of a lost spin
+            recorded = rec1.any();
+        }
     }
     // Without trajectories XYZ1 holds the last accepted position: the reference
     // stores every accepted position in place (kernels.cu:222-223), and a spin
     // that is lost keeps the one before.  Then the count of accepted steps.
+    // With trajectories a spin without a step shows its start (kernels.cu:95-99).
     const ArgsPtr c = cold(a);
-    if (!TRAJ) {
+    if (!TRAJ || (!recorded && c->traj_len)) {
         #pragma unroll
         for (int v = 0; v < NV; v++)
-            for (int i = 0; i < 3; i++) (SW_VIEW(c, xv, v, XYZ1) + xoff)[i] = PosVox::metres(*c, x[i], i);
+            for (int i = 0; i < 3; i++)
+                (SW_VIEW(c, xv, v, XYZ1) + xoff)[i] =
+                    TRAJ ? c->XYZ0[3 * (uint64_t)li + i] * c->xyz_scale : PosVox::metres(*c, x[i], i);
     }
     n_acc += (uint64_t)d * c->n_timepoints + tp;
     return st;
