@@ -213,12 +213,15 @@ SW_HD_INLINE uint32_t tissue_lds_words(const WalkArgs &a) {
     return a.tissue_lds ? a.n_sub * a.n_sub + 5 * a.n_sub : 0u;
 }
 
-// Staging in LDS, after a workgroup's tables: a ring of two 64-byte sectors of
-// recorded positions per lane.  Taken where it fits the 64 KiB of a workgroup and
-// kStageSpins rows or more are open (Recorder).
-constexpr uint32_t kStageBytes = 128, kStageSpins = 72u << 10;
+// Staging in LDS, after a workgroup's tables, where that fits the 64 KiB of a workgroup:
+// the next draws of a replayed spin's streams (ReplayRng), or a ring of two 64-byte
+// sectors of recorded positions where kStageSpins rows or more are open (Recorder).
+constexpr uint32_t kStageBytes = 128, kStageSpins = 72u << 10, kStageNormals = 24, kStageUniforms = 8;
+static_assert(4 * (kStageNormals + kStageUniforms) == kStageBytes, "one size for both");
 constexpr size_t stage_lds(uint32_t threads) { return (size_t)threads * kStageBytes + 16; }
-SW_HD_INLINE bool stage_wanted(const WalkArgs &a, bool replay) { return !replay && a.record_traj && a.n_local >= kStageSpins; }
+SW_HD_INLINE bool stage_wanted(const WalkArgs &a, bool replay) {
+    return replay || (a.record_traj && a.n_local >= kStageSpins);
+}
 
 // The kernel a walk takes.  Production walks of a scan with one TR, and those that
 // record trajectories, take the step loop of walk_prod.hpp; scans with dummy TRs

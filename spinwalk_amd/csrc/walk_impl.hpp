@@ -290,24 +290,63 @@ template <bool IDX32, class A> __device__ __forceinline__ uint32_t stage_ring(co
     return ((tables + 3) & ~3u) + (threadIdx.x >> 6) * (64 * kStageBytes / 4);
 }
 
-struct ReplayRng {          // the reference CPU path's recorded streams
+// the reference CPU path's recorded streams.  A spin's streams are rows of their own,
+// so a wave's lanes read from 64 places, and drawn one attempt at a time some lane
+// meets a line from HBM at nearly every step, which the wave waits for.  The draws
+// come kStageNormals and kStageUniforms at a time instead, into the lane's words in
+// LDS: one such wait for 8 attempts.  Spin echo of 401 time points on 40^3, 2e4 spins:
+// 0.92 -> 0.65 ms in FP32, 1.84 -> 0.66 ms in FP64; 2e5 spins of 80 steps on 96^3 0.69 -> 0.32
+// ms (compiled for 3 waves a SIMD at the same time: at 6 the positions in double
+// spilled, 76 registers of them; the streams leave no use for more waves).
+struct ReplayRng {
     static constexpr bool kReplay = true;
     const float *n, *u;
     uint64_t nn, nu, in = 0, iu = 0;
     float px = 0.f, py = 0.f, pz = 0.f;
     bool avail = false;
-    __device__ ReplayRng(const WalkArgs &a, uint32_t li, uint32_t) {
+    bool on;                        // staged (WalkArgs::stage)
+    uint32_t q;                     // the lane's words, 64 apart: axis_tab[q ..]
+    uint32_t at = kStageNormals, au = kStageUniforms;
+    typedef float Four __attribute__((ext_vector_type(4), aligned(4)));
+    __device__ ReplayRng(const WalkArgs &a, uint32_t li, uint32_t, uint32_t ring)
+        : on(a.stage), q(ring + (threadIdx.x & 63)) {
         n = a.rn + (uint64_t)li * a.rn_stride; nn = a.rn_stride;
         u = a.ru + (uint64_t)li * a.ru_stride; nu = a.ru_stride;
     }
+    // The next K words of a stream of `len`, from `i` on, into the words `first` ...
+    template <uint32_t K> __device__ void fill(const float *from, uint64_t i, uint64_t len, uint32_t first) {
+        if (i + K <= len) {
+            Four v[K / 4];
+            #pragma unroll
+            for (uint32_t k = 0; k < K / 4; k++) v[k] = *(GlobalPtr<Four>)(from + i + 4 * k);
+            #pragma unroll
+            for (uint32_t k = 0; k < K; k++) axis_tab[q + (first + k) * 64] = __float_as_uint(v[k / 4][k % 4]);
+        } else {
+            for (uint32_t k = 0; k < K && i + k < len; k++) axis_tab[q + (first + k) * 64] = __float_as_uint(from[i + k]);
+        }
+    }
     __device__ void peek() {
         avail = in + 3 <= nn;
-        if (avail) { px = n[in]; py = n[in + 1]; pz = n[in + 2]; }
+        if (!avail) return;
+        if (on) {
+            if (at == kStageNormals) { fill<kStageNormals>(n, in, nn, 0); at = 0; }
+            px = __uint_as_float(axis_tab[q + at * 64]);
+            py = __uint_as_float(axis_tab[q + (at + 1) * 64]);
+            pz = __uint_as_float(axis_tab[q + (at + 2) * 64]);
+        } else {
+            px = n[in]; py = n[in + 1]; pz = n[in + 2];
+        }
     }
-    __device__ void commit() { in += 3; }
+    __device__ void commit() { in += 3; at += 3; }
     __device__ bool uniform(float &v) {       // gen_u stream, one draw per substrate change
         if (iu >= nu) return false;
-        v = u[iu++];
+        if (on) {
+            if (au == kStageUniforms) { fill<kStageUniforms>(u, iu, nu, kStageNormals); au = 0; }
+            v = __uint_as_float(axis_tab[q + (kStageNormals + au++) * 64]);
+            iu++;
+        } else {
+            v = u[iu++];
+        }
         return true;
     }
 };
@@ -319,7 +358,7 @@ struct PhiloxRng {          // production: Philox4x32-10, one block per attempte
     float px = 0.f, py = 0.f, pz = 0.f;
     uint32_t pu = 0, ucur = 0;        // 24-bit permeability draws: next attempt's, last committed
     static constexpr bool avail = true;
-    __device__ PhiloxRng(const WalkArgs &a, uint32_t, uint32_t spin_global)
+    __device__ PhiloxRng(const WalkArgs &a, uint32_t, uint32_t spin_global, uint32_t = 0)
         : k0((uint32_t)a.seed), k1((uint32_t)(a.seed >> 32)) {
         const uint64_t m = (uint64_t)kPhiloxM1 * spin_global;
         m_hi = (uint32_t)(m >> 32);
@@ -816,7 +855,7 @@ __device__ int walk_spin(const WalkArgs &a, uint32_t li, uint64_t &n_acc, uint32
         tis.relax(ts_old, T1, T2);
     }
     uint32_t itr = 0;
-    Rng rng(a, li, spin);
+    Rng rng(a, li, spin, stage_ring<IDX32>(a));
     rng.peek();
     Phase ph;
     uint64_t slot = 0;
@@ -1072,7 +1111,7 @@ __device__ int walk_spin_views(const WalkArgs &a, const WalkView *xv, uint32_t l
         tis.relax(ts_old, T1, T2);
     }
     uint32_t itr = 0;
-    Rng rng(a, li, spin);
+    Rng rng(a, li, spin, stage_ring<IDX32>(a));
     rng.peek();
     Phase ph[NV];
     uint64_t slot = 0;
@@ -1514,6 +1553,9 @@ __device__ __forceinline__ void walk_block_views(const WalkArgs &a, const WalkVi
 }
 
 // Occupancy target: waves per SIMD the register allocation must allow.
+#ifndef SW_REPLAY_WAVES_PER_EU
+#define SW_REPLAY_WAVES_PER_EU 3
+#endif
 #ifndef SW_WALK_WAVES_PER_EU
 #define SW_WALK_WAVES_PER_EU 6
 #endif
@@ -1532,7 +1574,7 @@ __device__ __forceinline__ uint32_t single_position(uint32_t lanes, uint32_t blo
 }
 
 template <class Rng, class Rec, class Phase, bool CROSS, bool IDX32, bool PAIRS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIRS ? SW_PAIR_WAVES_PER_EU : SW_WALK_WAVES_PER_EU)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Rng::kReplay ? SW_REPLAY_WAVES_PER_EU : PAIRS ? SW_PAIR_WAVES_PER_EU : SW_WALK_WAVES_PER_EU)))
 void walk_kernel(const WalkArgs a) {
     // Blocks are dealt round-robin over the 8 XCDs; remap so that each XCD gets a
     // contiguous range of the visiting order (spatially sorted spins share L2).
@@ -1573,7 +1615,7 @@ constexpr int walk_waves_per_eu() {
 }
 
 template <class Rng, class Rec, class Phase, bool CROSS, bool IDX32, int NV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(walk_waves_per_eu<Phase, NV>())))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Rng::kReplay ? SW_REPLAY_WAVES_PER_EU : walk_waves_per_eu<Phase, NV>())))
 void walk_batch_kernel(const void *__restrict__ items, const BatchChunk *__restrict__ chunks, uint32_t spl) {
     const uint32_t per = gridDim.x / 8, b = blockIdx.x;
     const BatchChunk c = chunks[(b % 8) * per + b / 8];
@@ -1626,7 +1668,7 @@ template <class Rng, class F, class P, bool PAIRS>
 hipError_t launch_fp_loop(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
     const WalkMode m = mode_of<F>(a);
     const bool idx32 = m.idx32;
-    const size_t lds = capped_lds(a, idx32 ? m.lds : 0);
+    const size_t lds = capped_lds(a, (idx32 ? m.lds : 0) + (a.stage ? stage_lds(block.x) : 0));
     if constexpr (F::kPacked) {
         if (!idx32 && a.super_blocks) return hipErrorInvalidValue;   // super-blocks always fit the 32-bit mode
     }
