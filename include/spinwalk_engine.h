@@ -316,7 +316,8 @@ typedef struct sw_batch_schedule {
     uint32_t bands_shared;   /* bands per part when every tile of a class walks one phantom */
     uint32_t bands_mixed;    /* bands per part for the other classes                   */
     uint32_t spins_per_lane; /* 1 or 2: spins a lane walks, one after the other        */
-    uint32_t waves_per_simd; /* 0: as many as registers allow; 2-8: at most that many   */
+    uint32_t waves_per_simd; /* 0: as many as registers allow; 2-8: at most that many
+                                (sw_batch_create starts large batches with 4 or 5)      */
     uint32_t order_brick;    /* 4, 8, 16 or 32 voxels                                  */
 } sw_batch_schedule;
 SW_API int  sw_batch_get_schedule(const sw_batch *b, sw_batch_schedule *out);

@@ -1035,6 +1035,7 @@ bool order_pays(const sw::WalkArgs &a, int field, bool replay) {
 // and do more per gather: 1000^3 with 2e6 spins 117.4 -> 109.0 ms, int16 400^3 (window
 // 8.4 MiB) 0.99, FP32 400^3 (17 MiB) 1.13.
 constexpr uint64_t kWaveSpins = 64 * 1024;               // a wave on each of the 1024 SIMDs
+constexpr uint32_t kBatchWaves = 5;
 constexpr double kCapWindow = 2.8 * (1 << 20), kCapWindowFused = 12. * (1 << 20);
 bool cap_pays(uint64_t rec_bytes, uint64_t n_tile, uint64_t n_all, bool sorted, bool fused) {
     double window = (double)rec_bytes;
@@ -1600,7 +1601,11 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         SW_HIP(e, hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
         b->lds_block = (size_t)v;
     }
-    // capped where that pays for the walks that make up more than half of the spin-steps
+    // Capped at kCapWaves where that pays for the walks that make up more than half of
+    // the spin-steps, else at 5 where there are 6 waves a SIMD: tiles of a batch share no
+    // lines, and the sixth wave costs the others more than it brings.  Uncapped time over
+    // that at 5: 12 phantoms 1.07 (FP32 and int16), 8 scales of 96^3 1.02 and 1.04, of 150^3
+    // 1.06 and 1.02, phase cycles of 200^3 1.07 and 1.04.
     sw_batch_schedule sched = kDefaultSchedule;
     uint64_t n_all = 0, all = 0, capped = 0;
     for (const auto &t : b->tiles) n_all += t.n_local;
@@ -1611,7 +1616,8 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         if (!x.record_traj && cap_pays(bytes, t.n_local, n_all, x.order != nullptr, t.views > 1))
             capped += t.cost * t.n_local;
     }
-    if (b->rng != SW_RNG_REPLAY && 2 * capped > all) sched.waves_per_simd = sw::kCapWaves;
+    if (b->rng != SW_RNG_REPLAY && n_all >= 6 * kWaveSpins)
+        sched.waves_per_simd = 2 * capped > all ? sw::kCapWaves : kBatchWaves;
     int rc = apply_schedule(e, b.get(), sched, s, true);
     if (rc) return rc;
     *out = b.release();

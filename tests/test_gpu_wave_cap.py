@@ -36,7 +36,7 @@ def test_whole_equals_halves(engine, side, n, order, dummies):
         assert whole["stats"][k] == sum(p["stats"][k] for p in parts)
 
 
-@pytest.mark.parametrize("side,tiles,waves", [(190, 4, 4), (190, 3, 0), (96, 4, 0)])
+@pytest.mark.parametrize("side,tiles,waves", [(190, 4, 4), (190, 3, 0), (96, 4, 5), (96, 3, 0)])
 def test_default_schedule_of_a_batch(engine, side, tiles, waves):
     import torch
     m, f = cases.blocky_phantom((side,) * 3, n_labels=2, seed=side)
