@@ -992,7 +992,7 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
         if (o->step_loop == SW_STEP_LOOP_TWO) a.pairs = 1;
         else if (o->step_loop == SW_STEP_LOOP_AUTO) a.pairs = sw::walk_mode(a, field, 0).bytes > kPairsMinBytes ? 1u : 0u;
     }
-    // staging columns where the workgroup's 64 KiB of LDS hold them with the tables
+    // staging where the workgroup's 64 KiB of LDS hold it with the tables
     a.stage = sw::stage_wanted(a, o->rng == SW_RNG_REPLAY) && !a.pairs &&
               sw::walk_mode(a, field, o->rng == SW_RNG_REPLAY ? 1 : 0).lds + sw::stage_lds(256) <= 65536 ? 1u : 0u;
     return SW_OK;
@@ -1178,7 +1178,7 @@ struct sw_batch {
     std::vector<sw::ReduceItem> reduces;
     int rng = 0, field = 0, prec = 0;
     bool idx32 = false;
-    bool stage = false;                          // and staging columns (WalkArgs::stage)
+    bool stage = false;                          // some tile stages in LDS (WalkArgs::stage)
     bool mixed = false;                          // 64-bit mode over items in both packed layouts
     size_t lds = 0;                              // LDS of a workgroup: per-axis tables, then tissue tables (32-bit mode)
     // what the chunk table is built from: per walk unit (a single tile, or a
@@ -1207,7 +1207,7 @@ struct sw_batch {
 namespace {
 
 // Counter reset, the walk of every group and the echo sums, in stream order.
-// The LDS of a batch workgroup: the per-axis tables, raised so that at most
+// The LDS of a batch workgroup: the tables and the staging, raised so that at most
 // waves_per_simd waves fit each SIMD when the schedule asks for a cap.  A CU
 // has 4 SIMDs and a workgroup chunk_spins / 64 waves, so the cap is
 // k = 256 * waves_per_simd / chunk_spins workgroups per CU; k fit when
