@@ -534,8 +534,7 @@ static int phantom_finish(sw_engine *e, sw_phantom *ph, uint32_t formats) {
         SW_HIP(e, sw::launch_records(ph->mask, ph->field, nx, ny, nz, kind,
                                      1.0f / (f == SW_FIELD_Q16 ? ph->q_scale : ph->half_scale), ph->rec[f], s));
         if (f == SW_FIELD_F32) {         // the production walks' copies: packed for batches, SoA for single walks
-            SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, false, ph->rec_packed, s));
-            SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, true, ph->rec_soa, s));
+            SW_HIP(e, sw::launch_f32_records(ph->mask, ph->field, nx, ny, nz, ph->rec_packed, ph->rec_soa, s));
         }
     }
     SW_HIP(e, hipStreamSynchronize(s));

@@ -85,11 +85,12 @@ __device__ __forceinline__ uint32_t field16(float field, float inv_scale) {
 // Row-major mask/field -> bricked records (walk_args.hpp).  One thread builds one
 // 128-byte line, a brick, in registers and writes it whole, padding included, so
 // the array needs no clearing; neighbouring lanes take bricks neighbouring in z,
-// so their reads of a row of voxels are contiguous.  (One thread per voxel, its
+// so their reads of a row of voxels are contiguous.  The two float32 copies of the
+// production walks have the same bricks and are built together.  (One thread per voxel, its
 // record written byte by byte into a cleared array, took 104 us a copy at 256^3
-// for the float32 formats; this takes 55 us, 5 B read and 5.3 or 8 B written a voxel,
-// 3.1 to 4 TB/s.)
-enum : int { REC_F32 = 0, REC_F16 = 1, REC_BF16 = 2, REC_NONE = 3, REC_Q16 = 4, REC_PACKED = 5, REC_SOA = 6 };
+// for the float32 formats; this takes 55 us for the 8-byte records, 5 B read and 8 B
+// written a voxel, 4 TB/s, and 87 us for the two copies, 110 us one by one.)
+enum : int { REC_F32 = 0, REC_F16 = 1, REC_BF16 = 2, REC_NONE = 3, REC_Q16 = 4, REC_F32_PAIR = 5 };
 template <int KIND> struct BrickOf {         // voxels of a line per axis
     static constexpr bool k16 = KIND == REC_F16 || KIND == REC_BF16 || KIND == REC_Q16;
     static constexpr int bx = KIND == REC_F32 ? 1 << kBrick8.lbx : KIND == REC_NONE ? 1 << kBrick4.lbx : k16 ? kPack16.bx : kPackF32.bx;
@@ -108,13 +109,13 @@ __device__ __forceinline__ void put_bytes(uint32_t w[32], int at, uint32_t v, in
 template <int KIND>
 __global__ __launch_bounds__(256) void bricks_kernel(const uint8_t *mask, const float *field, uint32_t nx, uint32_t ny,
                                                      uint32_t nz, uint32_t n_x, uint32_t n_y, uint32_t n_z, uint64_t nb_y,
-                                                     uint64_t nb_z, bool sup, float inv_scale, uint4 *out) {
+                                                     uint64_t nb_z, bool sup, float inv_scale, uint4 *out, uint4 *out2) {
     using B = BrickOf<KIND>;
     const uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (id >= (uint64_t)n_x * n_y * n_z) return;
     const uint32_t id32 = (uint32_t)id;                                // below 2^32: 512 GiB of lines
     const uint32_t gz = id32 % n_z, gy = (id32 / n_z) % n_y, gx = id32 / n_z / n_y;
-    uint32_t w[32] = {};
+    uint32_t w[32] = {}, w2[KIND == REC_F32_PAIR ? 32 : 1] = {};
     #pragma unroll
     for (int x = 0; x < B::bx; x++)
         #pragma unroll
@@ -131,8 +132,10 @@ __global__ __launch_bounds__(256) void bricks_kernel(const uint8_t *mask, const 
                 const int j = (x * B::by + y) * B::bz + z;
                 if (KIND == REC_F32) { w[2 * j] = __float_as_uint(f); w[2 * j + 1] = lab; }
                 else if (KIND == REC_NONE) w[j] = lab << 16;
-                else if (KIND == REC_PACKED) { put_bytes(w, 5 * j, lab, 1); put_bytes(w, 5 * j + 1, __float_as_uint(f), 4); }
-                else if (KIND == REC_SOA) { put_bytes(w, j, lab, 1); w[kSoaF32.nvox / 4 + j] = __float_as_uint(f); }
+                else if (KIND == REC_F32_PAIR) {
+                    put_bytes(w, 5 * j, lab, 1); put_bytes(w, 5 * j + 1, __float_as_uint(f), 4);
+                    put_bytes(w2, j, lab, 1); w2[kSoaF32.nvox / 4 + j] = __float_as_uint(f);
+                }
                 else { put_bytes(w, 3 * j, lab, 1); put_bytes(w, 3 * j + 1, field16<KIND>(f, inv_scale), 2); }
             }
         }
@@ -140,11 +143,15 @@ __global__ __launch_bounds__(256) void bricks_kernel(const uint8_t *mask, const 
     const uint64_t line = kPacked ? pack_line(gx, gy, gz, nb_y, nb_z, sup) : ((uint64_t)gx * nb_y + gy) * nb_z + gz;
     #pragma unroll
     for (int k = 0; k < 8; k++) out[line * 8 + k] = make_uint4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+    if constexpr (KIND == REC_F32_PAIR) {
+        #pragma unroll
+        for (int k = 0; k < 8; k++) out2[line * 8 + k] = make_uint4(w2[4 * k], w2[4 * k + 1], w2[4 * k + 2], w2[4 * k + 3]);
+    }
 }
 
 template <int KIND>
 hipError_t launch_bricks(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz, float inv_scale,
-                         void *out, hipStream_t s) {
+                         void *out, hipStream_t s, void *out2 = nullptr) {
     using B = BrickOf<KIND>;
     uint64_t n_x, n_y, n_z, nb_y, nb_z;
     bool sup = false;
@@ -165,16 +172,15 @@ hipError_t launch_bricks(const uint8_t *mask, const float *field, uint64_t nx, u
     if (lines >= (1ull << 32)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(bricks_kernel<KIND>, dim3((unsigned)((lines + 255) / 256)), dim3(256), 0, s, mask, field,
                        (uint32_t)nx, (uint32_t)ny, (uint32_t)nz, (uint32_t)n_x, (uint32_t)n_y, (uint32_t)n_z, nb_y, nb_z,
-                       sup, inv_scale, (uint4 *)out);
+                       sup, inv_scale, (uint4 *)out, (uint4 *)out2);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_f32_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz,
-                              bool soa, void *out, hipStream_t s) {
-    return soa ? launch_bricks<REC_SOA>(mask, field, nx, ny, nz, 1.f, out, s)
-               : launch_bricks<REC_PACKED>(mask, field, nx, ny, nz, 1.f, out, s);
+                              void *packed, void *soa, hipStream_t s) {
+    return launch_bricks<REC_F32_PAIR>(mask, field, nx, ny, nz, 1.f, packed, s, soa);
 }
 
 hipError_t launch_phantom_stats(const uint8_t *mask, const float *field, uint64_t n, uint32_t *stats,

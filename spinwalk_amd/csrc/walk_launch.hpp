@@ -68,10 +68,10 @@ hipError_t launch_phantom_stats(const uint8_t *mask, const float *field, uint64_
 hipError_t launch_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz, int kind,
                           float inv_scale, void *out, hipStream_t s);
 // Row-major mask/field -> the float32 bricks of production walks: the packed
-// 5-byte records (kPackF32) batches gather, or with soa the structure-of-arrays
-// records (kSoaF32) single walks gather; every line of `out` is written, padding included.
+// 5-byte records (kPackF32) batches gather, and the structure-of-arrays records
+// (kSoaF32) single walks gather; every line of both is written, padding included.
 hipError_t launch_f32_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz,
-                              bool soa, void *out, hipStream_t s);
+                              void *packed, void *soa, hipStream_t s);
 // FP64 echo reduction into out[(te*n_sub+label)*3 + {0,1,2}].  partial is scratch
 // of reduce_partial_len(n, n_te, n_sub) doubles.
 struct ReduceItem {
