@@ -1171,7 +1171,7 @@ struct sw_batch {
     // the tiles' echo sums: one launch per pass over d_reduce, with scratch of every tile
     sw::ReduceItem *d_reduce = nullptr;
     double *d_partial = nullptr;
-    uint32_t reduce_blocks = 0, reduce_pairs = 0;
+    std::vector<sw::ReduceLaunch> reduce_launches;
     struct Group { int variant; int views; uint32_t offset, n_slots; };
     std::vector<Group> groups;
     std::vector<sw::ReduceItem> reduces;
@@ -1233,9 +1233,10 @@ hipError_t batch_enqueue(const sw_batch *b, hipStream_t s) {
                                     lds, s);
         if (err != hipSuccess) return err;
     }
-    if (!b->reduces.empty())
-        return sw::launch_echo_reduce_batch(b->d_reduce, (uint32_t)b->reduces.size(), b->reduce_blocks,
-                                            b->reduce_pairs, s);
+    for (const auto &l : b->reduce_launches) {
+        err = sw::launch_echo_reduce_batch(b->d_reduce, l, s);
+        if (err != hipSuccess) return err;
+    }
     return hipSuccess;
 }
 
@@ -1499,12 +1500,10 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
             r.M1 = it.d_M1; r.f64 = it.opts.precision == SW_PREC_F64; r.T = it.d_T;
             r.n = it.opts.n_local; r.n_te = it.sequence->n_te; r.n_sub = it.sequence->n_sub; r.out = it.d_echo_sums;
             if (r.n_te && r.n_sub) {
-                r.first_block = b->reduce_blocks;
-                r.first_pair = b->reduce_pairs;
-                b->reduce_blocks += sw::reduce_blocks(r.n, r.n_te, r.n_sub);
-                b->reduce_pairs += sw::reduce_pairs(r.n, r.n_te, r.n_sub);
+                if (!sw::reduce_plan(r))
+                    return fail(e, SW_E_INVALID, "tile " + std::to_string(i) + ": too many echoes and labels for the echo sums");
                 b->reduces.push_back(r);
-                partial += (size_t)sw::reduce_partial_len(r.n, r.n_te, r.n_sub);
+                partial += (size_t)sw::reduce_partial_len(r);
             }
         }
     }
@@ -1521,12 +1520,13 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
     SW_HIP(e, dev_upload(&b->d_exc, exc.data(), exc.size(), s));
     if (n_order) SW_HIP(e, hipMalloc((void **)&b->d_order, n_order * sizeof(uint32_t)));
     if (!b->reduces.empty()) {
-        SW_HIP(e, hipMalloc((void **)&b->d_partial, partial * sizeof(double)));
+        if (partial) SW_HIP(e, hipMalloc((void **)&b->d_partial, partial * sizeof(double)));
         size_t off = 0;
         for (auto &r : b->reduces) {
             r.partial = b->d_partial + off;
-            off += (size_t)sw::reduce_partial_len(r.n, r.n_te, r.n_sub);
+            off += (size_t)sw::reduce_partial_len(r);
         }
+        b->reduce_launches = sw::reduce_launches(b->reduces);
         SW_HIP(e, dev_upload(&b->d_reduce, b->reduces.data(), b->reduces.size(), s));
     }
     int rc0 = scratch_acquire(e, s);             // build_order_into uses the engine's sort scratch
@@ -1877,17 +1877,20 @@ SW_API int sw_echo_reduce_device(sw_engine *e, const void *d_M1, int m1_dtype, c
     SW_HIP(e, hipSetDevice(e->device));
     int rc = scratch_acquire(e, s);               // d_partial is engine-owned
     if (rc) return rc;
-    const size_t need = sw::reduce_partial_len(n_spins, n_te, n_sub);
+    sw::ReduceItem r{};
+    r.M1 = d_M1; r.T = d_T; r.out = d_out;
+    r.n = n_spins; r.n_te = n_te; r.n_sub = n_sub; r.f64 = m1_dtype == SW_DTYPE_F64;
+    if (!sw::reduce_plan(r)) return fail(e, SW_E_INVALID, "too many echoes and labels for the echo sums");
+    const size_t need = sw::reduce_partial_len(r);
     if (need > e->partial_cap) {
         SW_HIP(e, hipStreamSynchronize(s));
         dev_free(e->d_partial);
         e->d_partial = nullptr;
+        e->partial_cap = 0;
         SW_HIP(e, hipMalloc((void **)&e->d_partial, need * sizeof(double)));
         e->partial_cap = need;
     }
-    sw::ReduceItem r{};
-    r.M1 = d_M1; r.T = d_T; r.partial = e->d_partial; r.out = d_out;
-    r.n = n_spins; r.n_te = n_te; r.n_sub = n_sub; r.f64 = m1_dtype == SW_DTYPE_F64;
+    r.partial = e->d_partial;
     SW_HIP(e, sw::launch_echo_reduce(r, s));
     return scratch_release(e, s);
 }

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime_api.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "walk_args.hpp"
 
 namespace sw {
@@ -73,21 +75,24 @@ hipError_t launch_records(const uint8_t *mask, const float *field, uint64_t nx, 
 hipError_t launch_f32_records(const uint8_t *mask, const float *field, uint64_t nx, uint64_t ny, uint64_t nz,
                               void *packed, void *soa, hipStream_t s);
 // FP64 echo reduction into out[(te*n_sub+label)*3 + {0,1,2}].  partial is scratch
-// of reduce_partial_len(n, n_te, n_sub) doubles.
+// of reduce_partial_len doubles.
 struct ReduceItem {
     const void *M1;
     const uint8_t *T;
     double *partial, *out;
     uint32_t n, n_te, n_sub, f64;
-    uint32_t first_block, first_pair;      // the item's first of a batch's launches
+    uint32_t pieces, n_chunks, blocks, pairs;      // reduce_plan
+    uint32_t first_block, first_pair;              // the item's first of a batch's launch
 };
-uint64_t reduce_partial_len(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);
-uint32_t reduce_blocks(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);
-uint32_t reduce_pairs(uint32_t n_spins, uint32_t n_te, uint32_t n_sub);      // that need the second pass
+// Fills the plan of an item with its sizes; false where they are beyond a launch.
+bool reduce_plan(ReduceItem &r);
+uint64_t reduce_partial_len(const ReduceItem &r);
 hipError_t launch_echo_reduce(const ReduceItem &r, hipStream_t s);
-// Every item of items[] (device memory; n_blocks and n_pairs in all), one launch per pass.
-hipError_t launch_echo_reduce_batch(const ReduceItem *items, uint32_t n_items, uint32_t n_blocks, uint32_t n_pairs,
-                                    hipStream_t s);
+// A batch's items in device memory, one launch per pass for items [first, first + n_items):
+// reduce_launches gives the launches that hold them all (nearly always one).
+struct ReduceLaunch { uint32_t first, n_items, n_blocks, n_pairs; };
+std::vector<ReduceLaunch> reduce_launches(std::vector<ReduceItem> &items);
+hipError_t launch_echo_reduce_batch(const ReduceItem *items, const ReduceLaunch &l, hipStream_t s);
 
 // The fixed scratch of the no-allocation walk (noalloc.hip): its size, and the
 // device address of `device`'s copy, looked up once per device (`device` must
