@@ -1172,18 +1172,17 @@ struct sw_batch {
     sw::ReduceItem *d_reduce = nullptr;
     double *d_partial = nullptr;
     std::vector<sw::ReduceLaunch> reduce_launches;
-    struct Group { int variant; int views; uint32_t offset, n_slots; };
+    struct Group { int variant; int views; uint32_t offset, n_slots; bool stage; };
     std::vector<Group> groups;
     std::vector<sw::ReduceItem> reduces;
     int rng = 0, field = 0, prec = 0;
     bool idx32 = false;
-    bool stage = false;                          // some tile stages in LDS (WalkArgs::stage)
     bool mixed = false;                          // 64-bit mode over items in both packed layouts
     size_t lds = 0;                              // LDS of a workgroup: per-axis tables, then tissue tables (32-bit mode)
     // what the chunk table is built from: per walk unit (a single tile, or a
     // fused group of tiles), its kernel variant (launch_walk_batch), spins, steps
     // per spin, phantom records, views (1: d_items[index]; kMaxViews: d_fused[index])
-    struct Tile { int variant; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; };
+    struct Tile { int variant; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; bool stage; };
     std::vector<Tile> tiles;
     uint32_t n_fused_tiles = 0;                  // tiles walked inside fused units
     sw_batch_schedule sched{};
@@ -1205,14 +1204,13 @@ struct sw_batch {
 
 namespace {
 
-// Counter reset, the walk of every group and the echo sums, in stream order.
-// The LDS of a batch workgroup: the tables and the staging, raised so that at most
+// The LDS of a batch workgroup: the tables and its group's staging, raised so that at most
 // waves_per_simd waves fit each SIMD when the schedule asks for a cap.  A CU
 // has 4 SIMDs and a workgroup chunk_spins / 64 waves, so the cap is
 // k = 256 * waves_per_simd / chunk_spins workgroups per CU; k fit when
 // k * L <= LDS per CU < (k + 1) * L, so L = LDS per CU / (k + 1/2).
-size_t batch_lds(const sw_batch &b, const sw_batch_schedule &sc) {
-    size_t lds = (b.idx32 ? b.lds : 0) + (b.stage ? sw::stage_lds(sc.chunk_spins) : 0);
+size_t batch_lds(const sw_batch &b, const sw_batch_schedule &sc, bool stage) {
+    size_t lds = (b.idx32 ? b.lds : 0) + (stage ? sw::stage_lds(sc.chunk_spins) : 0);
     if (sc.waves_per_simd && b.lds_cu && sc.chunk_spins) {
         const size_t k = (size_t)256 * sc.waves_per_simd / sc.chunk_spins;
         const size_t l = (size_t)(2 * b.lds_cu / (2 * k + 1)) & ~(size_t)1023;
@@ -1221,16 +1219,23 @@ size_t batch_lds(const sw_batch &b, const sw_batch_schedule &sc) {
     return lds;
 }
 
+// Whether a schedule's LDS fits a workgroup in every group.
+bool batch_lds_ok(const sw_batch &b, const sw_batch_schedule &sc) {
+    for (const auto &t : b.tiles)
+        if (batch_lds(b, sc, t.stage) > b.lds_block) return false;
+    return true;
+}
+
+// Counter reset, the walk of every group and the echo sums, in stream order.
 hipError_t batch_enqueue(const sw_batch *b, hipStream_t s) {
     hipError_t err = sw::launch_zero_u64(b->d_counters, (int)(4 * b->n_items), s);
     if (err != hipSuccess) return err;
-    const size_t lds = batch_lds(*b, b->sched);
     for (const auto &g : b->groups) {
         const void *items = g.views == 1 ? (const void *)b->d_items : (const void *)b->d_fused;
         err = sw::launch_walk_batch(items, b->d_chunks + g.offset, g.n_slots, b->sched.chunk_spins,
                                     b->sched.spins_per_lane, g.views, b->rng, b->field, b->prec, g.variant,
                                     b->idx32 ? sw::ADDR_32 : b->mixed ? sw::ADDR_64_MIXED : sw::ADDR_64,
-                                    lds, s);
+                                    batch_lds(*b, b->sched, g.stage), s);
         if (err != hipSuccess) return err;
     }
     for (const auto &l : b->reduce_launches) {
@@ -1322,6 +1327,8 @@ void build_chunk_table(const sw_batch &b, const sw_batch_schedule &sc, std::vect
         sw_batch::Group g;
         g.variant = variant;
         g.views = views;
+        g.stage = false;
+        for (uint32_t i : idx) g.stage = g.stage || b.tiles[i].stage;
         g.offset = (uint32_t)table.size();
         g.n_slots = (uint32_t)(8 * per);
         for (auto &l : lists) {
@@ -1353,7 +1360,7 @@ int apply_schedule(sw_engine *e, sw_batch *b, const sw_batch_schedule &sc, hipSt
     std::vector<sw_batch::Group> groups;
     unsigned kinds = 0;
     build_chunk_table(*b, sc, table, groups, &kinds);
-    if (batch_lds(*b, sc) > b->lds_block)
+    if (!batch_lds_ok(*b, sc))
         return fail(e, SW_E_INVALID, "waves_per_simd " + std::to_string(sc.waves_per_simd) +
                                          " needs more LDS per workgroup than the device allows");
     // the previous table and orders may be in use by a run on any stream
@@ -1511,7 +1518,6 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
     // Tiles stage where the largest tile's tables leave the room.
     for (uint32_t i = 0; i < n_items; i++) {
         args[i].stage = sw::stage_wanted(args[i], b->rng == SW_RNG_REPLAY) && b->lds + sw::stage_lds(256) <= 65536;
-        b->stage = b->stage || args[i].stage;
     }
     for (uint32_t i = 0; i < n_items && !b->idx32; i++) b->mixed = b->mixed || args[i].super_blocks;
 
@@ -1564,7 +1570,7 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         const uint64_t cost = (uint64_t)(a0.n_dummy + 1) * a0.n_timepoints;
         const int variant = sw::walk_variant(a0, b->rng == SW_RNG_REPLAY);
         if (group.size() == 1) {
-            b->tiles.push_back({variant, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size()});
+            b->tiles.push_back({variant, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size(), a0.stage != 0});
             singles.push_back(a0);
             continue;
         }
@@ -1582,7 +1588,7 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
             w.M1 = x.M1; w.XYZ1 = x.XYZ1; w.T = x.T;
             w.counters = real ? x.counters : nullptr;      // a repeat of view 0 counts nothing
         }
-        b->tiles.push_back({variant, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size()});
+        b->tiles.push_back({variant, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size(), a0.stage != 0});
         fused.push_back(f);
         b->n_fused_tiles += (uint32_t)group.size();
     }
@@ -1748,7 +1754,7 @@ SW_API int sw_batch_tune(sw_batch *b, void *stream, uint32_t max_trials, sw_batc
     auto consider = [&](sw_batch_schedule cand) -> int {
         if (max_trials && trials >= max_trials) return SW_OK;
         if (std::memcmp(&cand, &best, sizeof cand) == 0) return SW_OK;
-        if (batch_lds(*b, cand) > b->lds_block) return SW_OK;     // a cap this device cannot express
+        if (!batch_lds_ok(*b, cand)) return SW_OK;     // a cap this device cannot express
         int r = timed(cand, &t);
         if (r) return r;
         if (t < 0.99f * t_best) { best = cand; t_best = t; }
