@@ -1,6 +1,6 @@
 """A batch of tiles of every kind: scans of one TR, scans with dummy TRs, recorded
 trajectories above and below the staging line, and fused tiles, each equal to its
-separate walk."""
+separate walk; scans with and without dummy TRs share one launch."""
 import numpy as np
 import pytest
 
@@ -45,4 +45,15 @@ def test_groups_equal_separate_walks(engine, kinds, mixed):
         st = b.run()
         for t, r, x in zip(tiles, refs, st["items"]):
             _check(t, r, x)
+    b.close()
+
+
+@pytest.mark.parametrize("kinds,launches", [(("ssfp", "ssfp"), 1), (("gre", "ssfp"), 1), (("gre", "gre", "few rows", "ssfp"), 1),
+                                            (("gre", "cross"), 1), (("cross", "gre", "ssfp"), 2), (("rows", "gre"), 2),
+                                            (("rows", "ssfp"), 2), (("few rows", "gre"), 1)])
+def test_launches(engine, kinds, launches):
+    """Graph nodes: counter reset, the walks, and the two passes of the echo sums."""
+    import torch
+    b = engine.batch(_tiles(engine, torch, kinds))
+    assert b.graph_info()["nodes"] == launches + 3
     b.close()
