@@ -22,6 +22,7 @@
 #include "../../include/spinwalk_engine.h"
 #include "walk_args.hpp"
 #include "walk_launch.hpp"
+#include "launch_rules.hpp"
 #include "phantom_gen.hpp"
 
 #define SW_VERSION_STRING "spinwalk-mi355x 0.1.0 (drop-in for SpinWalk 1.21.0 sim)"
@@ -159,6 +160,7 @@ struct sw_sequence {
     bool exc_valid = false;
     float key_lin = 0, key_quad = 0; int32_t key_ndummy = -1;
     float RF_FA0 = 0, RF_PH0 = 0;
+    double step_max = 0;             // metres per axis and step, of the tissue that diffuses fastest
     bool closed = false;             // no crossing probability between two tissues is above 0
     // The tables that shape a walk's trajectory and relaxation, byte for byte:
     // diffusivity, P_XY, T1/T2 and every event time.  Tiles whose sequences have
@@ -758,6 +760,7 @@ SW_API int sw_sequence_create(sw_engine *e, const sw_params *p, const sw_seq *q,
         T1d[i] = (double)q->T1_ms[i] * 1e-3;
         T2d[i] = (double)q->T2_ms[i] * 1e-3;
     }
+    for (uint32_t i = 0; i < ns; i++) sq->step_max = std::max(sq->step_max, fabs(q->diffusivity[i]));
     sq->closed = true;
     for (uint32_t i = 0; i < ns; i++)
         for (uint32_t j = 0; j < ns; j++)
@@ -863,17 +866,6 @@ int build_order(sw_engine *e, const sw::WalkArgs &a, hipStream_t s) {
     }
     return build_order_into(e, a, e->d_order, s);
 }
-
-// Spins per wave of a single walk.  A wave takes as long as the slowest of its lanes,
-// the one that meets the most vessel walls and redraws, and a SIMD with one wave waits
-// out every latency of it.  So where waves of half as many spins still find a SIMD
-// each, half the lanes stay empty, 64 lanes against 32: 64^3, GRE of 400 steps, 1e3
-// spins 260 -> 238 us, 3.2e4 302 -> 275; 256^3, 3e2 spins 182 -> 184 us, 2e3 219 -> 214,
-// 3.2e4 288 -> 263; bSSFP of 20 dummies 1.38 -> 1.25 ms at 8e3; replayed spin echo of
-// 2e4 spins 1.26 -> 0.93 ms.  Shorter waves lose again below 2 blocks a CU (8 lanes: 0.6 to
-// 0.75 of the rate of 64 at 1e3 spins), and above the line the waves share issue slots
-// (32 lanes 1.00 of the rate at 6.5e4 spins, 0.86 at 1e5).
-uint32_t single_lanes(uint32_t n_local) { return n_local <= 32u * 1024 ? 32 : 64; }
 
 // Checks one walk's arguments and fills its WalkArgs, except exc, order and
 // counters.  *field_out receives the record format the walk gathers.
@@ -985,7 +977,7 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
     // results).  Replayed walks and batches take one attempt per trip.
     if (o->step_loop < SW_STEP_LOOP_AUTO || o->step_loop > SW_STEP_LOOP_TWO)
         return fail(e, SW_E_INVALID, "unknown step_loop");
-    a.lanes = single_lanes(a.n_local);
+    a.lanes = sw::single_lanes(a.n_local);
     a.pairs = 0;
     if (o->rng == SW_RNG_PHILOX) {
         if (o->step_loop == SW_STEP_LOOP_TWO) a.pairs = 1;
@@ -1001,20 +993,14 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
 
 namespace {
 
-// Whether a single walk that asks for spatial order gets it.  Sorted spins share
-// lines with their neighbours, which pays when more spins are in flight than the
-// L2s (8 of 4 MiB in 128-byte lines: 262144) hold lines for, each its own.  Below
-// that every spin keeps its line by itself, and order only costs: its launches, and
-// waves of neighbours, some of which all meet vessel walls and redraw while others
-// are long done.  The same when the records fit each L2.  Sorted time over unsorted
-// (800 steps, FP32): 256^3 1.20 at 6.5e4 spins, 1.18 at 1.3e5, 0.98 to 1.10 at 2e5, 0.74
-// to 0.94 at 3e5, 0.52 at 1e6; 600^3 1.14 at 1.3e5, 1.10 at 2.1e5; int16 records of
-// 200^3 1.22 at 1.3e5, 1.04 at 2.4e5, 0.84 at 3e5; 64^3, whose records fit, 1.35 at 1.3e5
-// and 1.25 at 5e5.  PGSE trains on packed axons 0.98 to 1.04 at 6e4 to 2.1e5.
-constexpr uint32_t kUnsortedSpins = 208u << 10;
-constexpr uint64_t kUnsortedBytes = 4ull << 20;
-bool order_pays(const sw::WalkArgs &a, int field, bool replay) {
-    return a.n_local > kUnsortedSpins && sw::walk_mode(a, field, replay ? 1 : 0).bytes >= kUnsortedBytes;
+// The step of a walk, in voxels: the standard deviation along one axis, of the tissue
+// that diffuses fastest, along the axis of the smallest voxels.
+double voxel_step(const sw_sequence &q, const sw::WalkArgs &a) {
+    return q.step_max * std::max({a.s2g[0], a.s2g[1], a.s2g[2]});
+}
+
+bool order_pays(const sw_sequence &q, const sw::WalkArgs &a, int field, bool replay) {
+    return sw::order_pays(a.n_local, sw::walk_mode(a, field, replay ? 1 : 0).bytes, voxel_step(q, a));
 }
 
 // Whether the waves on a SIMD are held to kCapWaves.  Each spin in flight comes
@@ -1068,7 +1054,7 @@ SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence 
     a.exc = q->exc;
     a.counters = e->d_counters;
     a.order = nullptr;
-    if (o->spatial_order && order_pays(a, field, o->rng == SW_RNG_REPLAY)) {
+    if (o->spatial_order && order_pays(*q, a, field, o->rng == SW_RNG_REPLAY)) {
         rc = build_order(e, a, s);
         if (rc) return rc;
         a.order = e->d_order;
@@ -1130,7 +1116,7 @@ SW_API int sw_walk_device_noalloc(sw_engine *e, const sw_phantom *ph, const sw_s
                                              std::to_string(256 + order_bytes + plan.total_bytes) +
                                              " bytes of scratch; the no-allocation scratch holds " +
                                              std::to_string(cap) + " (use spatial_order 0 or sw_walk_device)");
-        if (order_pays(a, field, o->rng == SW_RNG_REPLAY)) {
+        if (order_pays(*q, a, field, o->rng == SW_RNG_REPLAY)) {
             uint32_t *order = (uint32_t *)(base + 256);
             SW_HIP(e, sw::launch_spatial_order(plan, base + 256 + order_bytes, a.XYZ0, a.xyz_scale, o->n_local, a.s2g,
                                                a.nx, a.ny, a.nz, order, s));
