@@ -994,44 +994,30 @@ int fill_walk_args(sw_engine *e, const sw_phantom *ph, const sw_sequence *q, con
 namespace {
 
 // The step of a walk, in voxels: the standard deviation along one axis, of the tissue
-// that diffuses fastest, along the axis of the smallest voxels.
-double voxel_step(const sw_sequence &q, const sw::WalkArgs &a) {
-    return q.step_max * std::max({a.s2g[0], a.s2g[1], a.s2g[2]});
+// that diffuses fastest, along the axis of the smallest (or largest) voxels.
+double voxel_step(const sw_sequence &q, const sw::WalkArgs &a, bool smallest) {
+    const double s2g = smallest ? std::max({a.s2g[0], a.s2g[1], a.s2g[2]}) : std::min({a.s2g[0], a.s2g[1], a.s2g[2]});
+    return q.step_max * s2g;
 }
 
 bool order_pays(const sw_sequence &q, const sw::WalkArgs &a, int field, bool replay) {
-    return sw::order_pays(a.n_local, sw::walk_mode(a, field, replay ? 1 : 0).bytes, voxel_step(q, a));
+    return sw::order_pays(a.n_local, sw::walk_mode(a, field, replay ? 1 : 0).bytes, voxel_step(q, a, true));
 }
 
-// Whether the waves on a SIMD are held to kCapWaves.  Each spin in flight comes
-// back to the line it last read; the waves that fit a SIMD (8) hold twice the lines
-// of an L2, kCapWaves half of one XCD's, so fewer waves wait less.  It pays when
-//  - the records the spins in flight meet exceed an L2 (kCapWindow): the whole
-//    phantom when unsorted, an eighth (an XCD's part) when sorted, and of it the
-//    share of its spins that 8 waves are;
-//  - there are 6 waves a SIMD or more, so that the last round is not a fraction of
-//    the others (4 and a bit waves would take two rounds for one).
-// Uncapped time over capped, single walks: FP32 records of 256^3
-// 1.26 at 4e5 spins, 1.15 at 5e5, 1.10 at 1e6, 1.03 at 1.5e6; 400^3 1.08; 128^3 (window
-// 1 MiB) 0.95 to 0.99, so not capped.  int16 records of 400^3 1.54 at 5e5, 1.37 at 8e5
-// (bSSFP), 1.13 at 1.5e6; of 256^3 1.18 at 4e5, 1.02 at 7e5, 0.99 at 8e5 (window 2.7).
-// 3e5 spins (4.6 waves) 0.82 to 0.88 on 256^3.  Batches: 32 scales of 256^3, 1e5 spins
-// each, 116.7 -> 95.7 ms; 200^3 int16 0.95 fused.  Fused walks, which hold 5 waves anyway
-// and do more per gather: 1000^3 with 2e6 spins 117.4 -> 109.0 ms, int16 400^3 (window
-// 8.4 MiB) 0.99, FP32 400^3 (17 MiB) 1.13.
-constexpr uint64_t kWaveSpins = 64 * 1024;               // a wave on each of the 1024 SIMDs
-constexpr uint32_t kBatchWaves = 5;
-constexpr double kCapWindow = 2.8 * (1 << 20), kCapWindowFused = 12. * (1 << 20);
-bool cap_pays(uint64_t rec_bytes, uint64_t n_tile, uint64_t n_all, bool sorted, bool fused) {
-    double window = (double)rec_bytes;
-    if (sorted) window *= std::min(1., 8. * (double)kWaveSpins / (double)n_tile) / 8;
-    return n_all >= 6 * kWaveSpins && window > (fused ? kCapWindowFused : kCapWindow);
+bool cap_pays(sw::CapKind kind, const sw_sequence &q, const sw::WalkArgs &a, int field, uint64_t n_all) {
+    const uint64_t bytes = sw::walk_mode(a, field, 0).bytes;
+    const double voxels = (double)a.matrix_length, steps = (double)(a.n_dummy + 1) * a.n_timepoints;
+    const bool sorted = a.order != nullptr;
+    return sw::cap_pays(kind, a.n_dummy == 0,
+                        sw::cap_reach(bytes, voxels, a.n_local, sorted, voxel_step(q, a, false), steps),
+                        sw::cap_window(bytes, voxels, a.n_local, sorted, 0.), n_all);
 }
+
+constexpr uint32_t kBatchWaves = 5;
 
 // Trajectories and replayed draws stream from HBM and keep every wave they can.
-uint32_t single_cap(const sw::WalkArgs &a, int field, bool replay) {
-    return !replay && !a.record_traj &&
-           cap_pays(sw::walk_mode(a, field, 0).bytes, a.n_local, a.n_local, a.order != nullptr, false);
+uint32_t single_cap(const sw_sequence &q, const sw::WalkArgs &a, int field, bool replay) {
+    return !replay && !a.record_traj && cap_pays(a.pairs ? sw::CAP_PAIRS : sw::CAP_SINGLE, q, a, field, a.n_local);
 }
 
 }  // namespace
@@ -1059,7 +1045,7 @@ SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence 
         if (rc) return rc;
         a.order = e->d_order;
     }
-    a.cap = single_cap(a, field, o->rng == SW_RNG_REPLAY);
+    a.cap = single_cap(*q, a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(e->d_counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
     SW_HIP(e, sw::launch_walk(a, o->rng == SW_RNG_REPLAY ? 1 : 0, field, o->precision, s));
@@ -1123,7 +1109,7 @@ SW_API int sw_walk_device_noalloc(sw_engine *e, const sw_phantom *ph, const sw_s
             a.order = order;
         }
     }
-    a.cap = single_cap(a, field, o->rng == SW_RNG_REPLAY);
+    a.cap = single_cap(*q, a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(a.counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
     SW_HIP(e, sw::launch_walk(a, o->rng == SW_RNG_REPLAY ? 1 : 0, field, o->precision, s));
@@ -1168,7 +1154,7 @@ struct sw_batch {
     // what the chunk table is built from: per walk unit (a single tile, or a
     // fused group of tiles), its kernel variant (launch_walk_batch), spins, steps
     // per spin, phantom records, views (1: d_items[index]; kMaxViews: d_fused[index])
-    struct Tile { int variant; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; bool stage; };
+    struct Tile { int variant; uint32_t n_local; uint64_t cost; const void *rec; int views; uint32_t index; bool stage; uint32_t item; };
     std::vector<Tile> tiles;
     uint32_t n_fused_tiles = 0;                  // tiles walked inside fused units
     sw_batch_schedule sched{};
@@ -1556,7 +1542,7 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         const uint64_t cost = (uint64_t)(a0.n_dummy + 1) * a0.n_timepoints;
         const int variant = sw::walk_variant(a0, b->rng == SW_RNG_REPLAY);
         if (group.size() == 1) {
-            b->tiles.push_back({variant, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size(), a0.stage != 0});
+            b->tiles.push_back({variant, a0.n_local, cost, a0.rec, 1, (uint32_t)singles.size(), a0.stage != 0, i});
             singles.push_back(a0);
             continue;
         }
@@ -1574,7 +1560,7 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
             w.M1 = x.M1; w.XYZ1 = x.XYZ1; w.T = x.T;
             w.counters = real ? x.counters : nullptr;      // a repeat of view 0 counts nothing
         }
-        b->tiles.push_back({variant, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size(), a0.stage != 0});
+        b->tiles.push_back({variant, a0.n_local, cost, a0.rec, sw::kMaxViews, (uint32_t)fused.size(), a0.stage != 0, i});
         fused.push_back(f);
         b->n_fused_tiles += (uint32_t)group.size();
     }
@@ -1619,21 +1605,21 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
         b->lds_block = (size_t)v;
     }
     // Capped at kCapWaves where that pays for the walks that make up more than half of
-    // the spin-steps, else at 5 where there are 6 waves a SIMD: tiles of a batch share no
-    // lines, and the sixth wave costs the others more than it brings.  Uncapped time over
+    // the spin-steps, else at 5 where there are 6 waves a SIMD: the sixth wave's lines cost
+    // the others more than it brings.  Uncapped time over
     // that at 5: 12 phantoms 1.07 (FP32 and int16), 8 scales of 96^3 1.02 and 1.04, of 150^3
-    // 1.06 and 1.02, phase cycles of 200^3 1.07 and 1.04.
+    // 1.06 and 1.02, phase cycles of 200^3 1.07 and 1.04; recorded trajectories 0.99 to 1.03.
     sw_batch_schedule sched = kDefaultSchedule;
     uint64_t n_all = 0, all = 0, capped = 0;
     for (const auto &t : b->tiles) n_all += t.n_local;
     for (const auto &t : b->tiles) {
         const sw::WalkArgs &x = t.views == 1 ? singles[t.index] : fused[t.index].a;
-        const uint64_t bytes = sw::walk_mode(x, b->field, b->rng == SW_RNG_REPLAY ? 1 : 0).bytes;
         all += t.cost * t.n_local;
-        if (!x.record_traj && cap_pays(bytes, t.n_local, n_all, x.order != nullptr, t.views > 1))
+        if (!x.record_traj &&
+            cap_pays(t.views > 1 ? sw::CAP_FUSED : sw::CAP_BATCH, *items[t.item].sequence, x, b->field, n_all))
             capped += t.cost * t.n_local;
     }
-    if (b->rng != SW_RNG_REPLAY && n_all >= 6 * kWaveSpins)
+    if (b->rng != SW_RNG_REPLAY && n_all >= 6 * sw::kWaveSpins)
         sched.waves_per_simd = 2 * capped > all ? sw::kCapWaves : kBatchWaves;
     int rc = apply_schedule(e, b.get(), sched, s, true);
     if (rc) return rc;

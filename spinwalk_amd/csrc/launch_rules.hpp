@@ -1,11 +1,15 @@
 // launch_rules.hpp -- how a walk is launched, as rules on its sizes: whether its spins
-// are visited sorted and how many a wave carries.  None changes a result.  Plain C++.
+// are visited sorted, how many a wave carries, and whether the waves on a SIMD are
+// capped.  None changes a result.  Plain C++.
 #pragma once
+#include <math.h>
 #include <stdint.h>
 
 #include <algorithm>
 
 namespace sw {
+
+constexpr uint64_t kWaveSpins = 64 * 1024;               // a wave on each of the 1024 SIMDs
 
 // Spins per wave of a single walk.  A wave takes as long as the slowest of its lanes,
 // the one that meets the most vessel walls and redraws, and a SIMD with one wave waits
@@ -45,6 +49,51 @@ inline uint32_t unsorted_spins(double step) {
 }
 inline bool order_pays(uint32_t n_local, uint64_t rec_bytes, double step) {
     return n_local > unsorted_spins(step) && rec_bytes >= kUnsortedBytes;
+}
+
+// Whether the waves on a SIMD are held to kCapWaves (4) in a single walk, or a batch's to
+// 4 and not 5.  Each spin in flight comes back to the lines it last read; the waves that
+// fit a SIMD (8) hold more lines than an L2, so fewer waves wait less.  What they wait
+// for grows with
+//  - the records that the spins in flight on an XCD meet: of the whole phantom when
+//    unsorted, of an eighth when sorted (an XCD's part), of it the share of its spins
+//    that 8 waves are, and around it what spins drift over the walk;
+//  - the step (in voxels): how often a spin needs another line, and of how many.
+// cap_reach is the product, MiB voxel^2.  The lines are where uncapped and capped time
+// cross over 80^3 to 500^3, steps of 0.1 to 2.5, 160 to 5100 time points, float32 and int16
+// records, 4e5 to 2e6 spins.  Uncapped time over capped (for a batch, 5 waves over 4),
+// nine tenths of the measurements below and above the line:
+//                       line   below          above
+//   one TR              0.85   0.92 to 1.12   0.98 to 1.49   (FP32 256^3, step 0.32, 800 points: 1.26 at 4e5 spins)
+//   dummy TRs           1.1    0.92 to 1.02   0.96 to 1.49
+//   two attempts        1.85   0.92 to 1.00   0.99 to 1.11   (a trip of the loop: records above 256 MiB; 500^3, 1e6
+//                                                             spins of a spin echo of 2000 points 1.02)
+//     with dummy TRs    2.5    0.93 to 0.98   0.98 to 1.14
+//   batch, dummy TRs    8      0.88 to 1.01   0.95 to 1.23
+//   fused, one TR       1.2    0.91 to 1.06   0.99 to 1.34
+//   fused, dummy TRs    2.1    0.89 to 1.03   0.96 to 1.35   (1000^3 with 2e6 spins 117.4 -> 109.0 ms)
+// A batch of scans with one TR goes by the records alone (kCapWindow, without drift): its
+// tiles of one phantom meet in the same lines where few are in flight.  The FoV sweep's 64
+// tiles, whose reach is 0 to 8, run 95.3 ms at 4 waves and 104.2 at 5; six tiles of one scale
+// 0.90 to 0.97 below a reach of 2, 0.94 to 1.16 above.
+// Only from 6 waves a SIMD on, so that the last round is not a fraction of the others: 3e5
+// spins (4.6 waves) 0.82 to 0.88 on 256^3.
+enum CapKind : int { CAP_SINGLE = 0, CAP_PAIRS = 1, CAP_BATCH = 2, CAP_FUSED = 3 };
+constexpr double kCapWindow = 2.8;
+// The records in reach, MiB; drift: how far spins spread over the walk, in voxels.
+inline double cap_window(uint64_t rec_bytes, double voxels, uint64_t n_tile, bool sorted, double drift) {
+    const double part = sorted ? std::min(1., 8. * (double)kWaveSpins / (double)n_tile) / 8 : 1.;
+    const double side = cbrt(voxels * part) + 0.7 * drift;           // 0.35 standard deviations each way
+    return (double)rec_bytes / (1 << 20) * std::min(1., side * side * side / voxels);
+}
+inline double cap_reach(uint64_t rec_bytes, double voxels, uint64_t n_tile, bool sorted, double step, double n_steps) {
+    const double often = std::min(step, 0.65);           // longer steps meet another line every time
+    return cap_window(rec_bytes, voxels, n_tile, sorted, step * sqrt(n_steps)) * often * often;
+}
+inline bool cap_pays(CapKind kind, bool one_tr, double reach, double window, uint64_t n_all) {
+    constexpr double kLine[4][2] = {{1.1, 0.85}, {2.5, 1.85}, {8., 0.}, {2.1, 1.2}};
+    if (n_all < 6 * kWaveSpins) return false;
+    return kind == CAP_BATCH && one_tr ? window > kCapWindow : reach > kLine[kind][one_tr];
 }
 
 }  // namespace sw

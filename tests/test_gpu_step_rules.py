@@ -1,9 +1,11 @@
 """Spins of long steps are visited sorted from fewer spins on, with the results of a
-walk without order."""
+walk without order, and batches of scans with dummy TRs start with 5 waves a SIMD
+where scans of one TR start with 4."""
 import numpy as np
 import pytest
 
 from tests import cases
+from tests.test_gpu_batch import _tile
 from tests.test_gpu_production import run
 
 pytestmark = pytest.mark.gpu
@@ -18,3 +20,17 @@ def test_sorted_equals_unsorted(engine, n):
         np.testing.assert_array_equal(a[k], b[k])
     for k in ("n_lost", "n_steps", "n_attempts"):
         assert a["stats"][k] == b["stats"][k]
+
+
+@pytest.mark.parametrize("dummies,waves", [(0, 4), (4, 5)])
+def test_default_waves_of_a_batch(engine, dummies, waves):
+    import torch
+    m, f = cases.blocky_phantom((190,) * 3, n_labels=2, seed=3)
+    case = cases.make_case(cases.gre(2, TE=200, dt=50, DUMMY_SCAN=dummies), m, f, 90.0, n_spins=100000)
+    ph = engine.phantom(case.mask, case.field_T, case.fov)
+    items = [_tile(engine, torch, case, ph=ph) for _ in range(4)]
+    for k, t in enumerate(items):
+        t["params"].seed = 10 + k                          # tiles of one seed would fuse
+    b = engine.batch(items)
+    assert b.schedule["waves_per_simd"] == waves
+    b.close()
