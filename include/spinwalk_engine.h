@@ -129,6 +129,11 @@ typedef struct sw_walk_stats {
  * (src/sim/monte_carlo.cu:33-55) + check_CUDA (src/sim/device_helper.cu:18-30). */
 SW_API int  sw_engine_create(int device_id, sw_engine **out);
 SW_API void sw_engine_destroy(sw_engine *eng);
+/* An engine keeps the device memory of destroyed phantoms (up to 4 blocks, 2 GiB
+ * together) for the next ones of a like size.  It goes back when an allocation of any
+ * engine on the device does not fit beside it, with the engine, and by this call: for a
+ * program that allocates device memory by other means. */
+SW_API int  sw_engine_trim(sw_engine *eng);
 SW_API const char *sw_last_error(const sw_engine *eng);
 /* print_device_info (src/sim/device_helper.cu:47-76): writes a text summary. */
 SW_API int  sw_device_info(int device_id, char *buf, size_t buflen);

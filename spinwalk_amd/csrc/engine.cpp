@@ -43,18 +43,21 @@ thread_local std::string g_tls_error;
 // back its memory each time cost more than preparing it (256^3, float32: 1.2 ms of
 // a 2.5 ms step; at higher rates the driver stalls whole calls by 10 ms).  At
 // most kBlocks blocks of kBytes in all; a block serves a phantom of its size or
-// down to half of it.  Given back when an allocation does not fit beside them and
-// with the engine; a phantom that outlives its engine frees its own.  Shared by
-// the engine and its phantoms, which may be destroyed from any thread.
+// down to 7/8 of it.  Given back when an allocation of any engine on the device does
+// not fit beside them (dev_malloc), by sw_engine_trim, and with the engine; a phantom
+// that outlives its engine frees its own.  Shared by the engine and its phantoms, which
+// may be destroyed from any thread.
 struct PhantomPool {
     static constexpr size_t kBlocks = 4, kBytes = 2ull << 30;
+    const int device;
+    explicit PhantomPool(int dev) : device(dev) {}
     std::mutex mu;
     bool open = true;
     std::vector<std::pair<void *, size_t>> kept;
     void *take(size_t bytes, size_t *got) {
         std::lock_guard<std::mutex> lock(mu);
         for (size_t i = 0; i < kept.size(); i++)
-            if (kept[i].second >= bytes && kept[i].second / 2 <= bytes) {
+            if (kept[i].second >= bytes && kept[i].second - kept[i].second / 8 <= bytes) {
                 void *p = kept[i].first;
                 *got = kept[i].second;
                 kept.erase(kept.begin() + i);
@@ -97,7 +100,7 @@ struct PhantomPool {
 };
 
 struct sw_engine {
-    std::shared_ptr<PhantomPool> pool = std::make_shared<PhantomPool>();
+    std::shared_ptr<PhantomPool> pool;
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
@@ -183,11 +186,58 @@ int fail(sw_engine *e, int code, const std::string &msg) {
             return fail((eng), SW_E_HIP, std::string(#expr) + ": " + hipGetErrorString(_e));  \
     } while (0)
 
+// The pools of the process's engines, for allocations that do not fit beside what they keep.
+std::mutex g_pools_mu;
+std::vector<std::weak_ptr<PhantomPool>> g_pools;
+
+std::shared_ptr<PhantomPool> make_pool(int device) {
+    auto p = std::make_shared<PhantomPool>(device);
+    std::lock_guard<std::mutex> lock(g_pools_mu);
+    g_pools.erase(std::remove_if(g_pools.begin(), g_pools.end(), [](const auto &w) { return w.expired(); }),
+                  g_pools.end());
+    g_pools.push_back(p);
+    return p;
+}
+
+// Gives back what the pools of `device` keep; false when that is nothing.
+bool release_pools(int device) {
+    std::vector<std::shared_ptr<PhantomPool>> pools;
+    {
+        std::lock_guard<std::mutex> lock(g_pools_mu);
+        for (const auto &w : g_pools)
+            if (auto p = w.lock()) pools.push_back(p);
+    }
+    bool any = false;
+    for (const auto &p : pools)
+        if (p->device == device && !p->empty()) {
+            p->release(false);
+            any = true;
+        }
+    return any;
+}
+
+// hipMalloc on the current device, once more without the pools' memory when it does
+// not fit beside it.
+hipError_t dev_malloc(void **p, size_t bytes) {
+    *p = nullptr;
+    hipError_t e = hipMalloc(p, bytes);
+    int device = 0;
+    if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && release_pools(device)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();                                 // reported here, not by the next launch
+        *p = nullptr;
+    }
+    return e;
+}
+
 template <class T>
 hipError_t dev_upload(T **dst, const T *src, size_t n, hipStream_t s) {
     *dst = nullptr;
     if (n == 0) return hipSuccess;
-    hipError_t e = hipMalloc((void **)dst, n * sizeof(T));
+    hipError_t e = dev_malloc((void **)dst, n * sizeof(T));
     if (e != hipSuccess) return e;
     if (src) return hipMemcpyAsync(*dst, src, n * sizeof(T), hipMemcpyHostToDevice, s);
     return hipSuccess;
@@ -253,7 +303,9 @@ int ensure_exc(sw_engine *e, sw_sequence *q, const sw_params *p, hipStream_t s) 
         SW_HIP(e, hipStreamSynchronize(s));
         dev_free(q->exc);
         q->exc = nullptr;
-        SW_HIP(e, hipMalloc((void **)&q->exc, n * sizeof(sw::Excitation)));
+        q->exc_cap = 0;
+        q->exc_valid = false;
+        SW_HIP(e, dev_malloc((void **)&q->exc, n * sizeof(sw::Excitation)));
         q->exc_cap = n;
     }
     SW_HIP(e, hipMemcpyAsync(q->exc, h.data(), n * sizeof(sw::Excitation), hipMemcpyHostToDevice, s));
@@ -268,10 +320,7 @@ int ensure_exc(sw_engine *e, sw_sequence *q, const sw_params *p, hipStream_t s) 
 int check_free_memory(sw_engine *e, size_t bytes) {   // device_helper.cu:78-101
     size_t fr = 0, tot = 0;
     SW_HIP(e, hipMemGetInfo(&fr, &tot));
-    if (bytes > fr && !e->pool->empty()) {
-        e->pool->release(false);
-        SW_HIP(e, hipMemGetInfo(&fr, &tot));
-    }
+    if (bytes > fr && release_pools(e->device)) SW_HIP(e, hipMemGetInfo(&fr, &tot));
     if (bytes > fr) {
         char b[256];
         snprintf(b, sizeof b, "not enough device memory: need %zu MB, free %zu MB", bytes >> 20, fr >> 20);
@@ -338,6 +387,7 @@ SW_API int sw_engine_create(int device_id, sw_engine **out) {
         return fail(nullptr, SW_E_NODEVICE, std::string("device is ") + pr.gcnArchName + ", this build targets gfx950");
     std::unique_ptr<sw_engine, void (*)(sw_engine *)> e(new sw_engine, sw_engine_destroy);
     e->device = device_id;
+    e->pool = make_pool(device_id);
     if (hipSetDevice(device_id) != hipSuccess) return fail(nullptr, SW_E_HIP, "hipSetDevice failed");
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(nullptr, SW_E_HIP, "hipStreamCreate failed");
@@ -360,7 +410,7 @@ SW_API void sw_engine_destroy(sw_engine *e) {
     dev_free(e->d_sort);
     dev_free(e->d_order);
     dev_free(e->d_partial);
-    e->pool->release(true);
+    if (e->pool) e->pool->release(true);
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->scratch_ev) {
@@ -488,16 +538,9 @@ static int phantom_alloc(sw_engine *e, sw_phantom *ph, uint32_t formats) {
     ph->arena = e->pool->take(total, &ph->arena_bytes);
     if (!ph->arena) {
         ph->arena_bytes = total;
-        hipError_t he = hipMalloc(&ph->arena, total);
-        if (he != hipSuccess && !e->pool->empty()) {         // again without what the pool holds
-            (void)hipGetLastError();
-            e->pool->release(false);
-            he = hipMalloc(&ph->arena, total);
-        }
-        if (he != hipSuccess) {
-            ph->arena = nullptr;
+        const hipError_t he = dev_malloc(&ph->arena, total);
+        if (he != hipSuccess)
             return fail(e, SW_E_HIP, std::string("hipMalloc of a phantom: ") + hipGetErrorString(he));
-        }
     }
     for (const auto &x : slices) *x.first = (char *)ph->arena + x.second;
     return SW_OK;
@@ -848,7 +891,8 @@ int build_order_into(sw_engine *e, const sw::WalkArgs &a, uint32_t *out, hipStre
         SW_HIP(e, hipStreamSynchronize(s));
         dev_free(e->d_sort);
         e->d_sort = nullptr;
-        SW_HIP(e, hipMalloc(&e->d_sort, plan.total_bytes));
+        e->sort_bytes = 0;
+        SW_HIP(e, dev_malloc(&e->d_sort, plan.total_bytes));
         e->sort_bytes = plan.total_bytes;
     }
     SW_HIP(e, sw::launch_spatial_order(plan, e->d_sort, a.XYZ0, a.xyz_scale, n, a.s2g, a.nx, a.ny, a.nz, out, s));
@@ -861,7 +905,8 @@ int build_order(sw_engine *e, const sw::WalkArgs &a, hipStream_t s) {
         SW_HIP(e, hipStreamSynchronize(s));
         dev_free(e->d_order);
         e->d_order = nullptr;
-        SW_HIP(e, hipMalloc((void **)&e->d_order, n * sizeof(uint32_t)));
+        e->order_cap = 0;
+        SW_HIP(e, dev_malloc((void **)&e->d_order, n * sizeof(uint32_t)));
         e->order_cap = n;
     }
     return build_order_into(e, a, e->d_order, s);
@@ -1354,7 +1399,7 @@ int apply_schedule(sw_engine *e, sw_batch *b, const sw_batch_schedule &sc, hipSt
         dev_free(b->d_chunks);
         b->d_chunks = nullptr;
         b->chunks_cap = 0;
-        SW_HIP(e, hipMalloc((void **)&b->d_chunks, table.size() * sizeof(sw::BatchChunk)));
+        SW_HIP(e, dev_malloc((void **)&b->d_chunks, table.size() * sizeof(sw::BatchChunk)));
         b->chunks_cap = table.size();
     }
     if (!table.empty())
@@ -1494,11 +1539,11 @@ SW_API int sw_batch_create(sw_engine *e, const sw_batch_item *items, uint32_t n_
     for (uint32_t i = 0; i < n_items && !b->idx32; i++) b->mixed = b->mixed || args[i].super_blocks;
 
     // ---- device tables
-    SW_HIP(e, hipMalloc((void **)&b->d_counters, 4 * n_items * sizeof(unsigned long long)));
+    SW_HIP(e, dev_malloc((void **)&b->d_counters, 4 * n_items * sizeof(unsigned long long)));
     SW_HIP(e, dev_upload(&b->d_exc, exc.data(), exc.size(), s));
-    if (n_order) SW_HIP(e, hipMalloc((void **)&b->d_order, n_order * sizeof(uint32_t)));
+    if (n_order) SW_HIP(e, dev_malloc((void **)&b->d_order, n_order * sizeof(uint32_t)));
     if (!b->reduces.empty()) {
-        if (partial) SW_HIP(e, hipMalloc((void **)&b->d_partial, partial * sizeof(double)));
+        if (partial) SW_HIP(e, dev_malloc((void **)&b->d_partial, partial * sizeof(double)));
         size_t off = 0;
         for (auto &r : b->reduces) {
             r.partial = b->d_partial + off;
@@ -1846,7 +1891,7 @@ SW_API int sw_walk_host(sw_engine *e, const sw_phantom *ph, const sw_sequence *q
         if (rc) return rc;
         for (int i = 0; i < 7; i++)
             if (bytes[i] > e->host_cap[i]) {
-                SW_HIP(e, hipMalloc(&e->d_host[i], bytes[i]));
+                SW_HIP(e, dev_malloc(&e->d_host[i], bytes[i]));
                 e->host_cap[i] = bytes[i];
             }
     }
@@ -1891,7 +1936,7 @@ SW_API int sw_echo_reduce_device(sw_engine *e, const void *d_M1, int m1_dtype, c
         dev_free(e->d_partial);
         e->d_partial = nullptr;
         e->partial_cap = 0;
-        SW_HIP(e, hipMalloc((void **)&e->d_partial, need * sizeof(double)));
+        SW_HIP(e, dev_malloc((void **)&e->d_partial, need * sizeof(double)));
         e->partial_cap = need;
     }
     r.partial = e->d_partial;
@@ -1921,6 +1966,13 @@ SW_API int sw_probe_gather_device(sw_engine *e, const void *d_buf, uint64_t byte
     SW_HIP(e, hipEventRecord(e->ev1, s));
     SW_HIP(e, hipEventSynchronize(e->ev1));
     SW_HIP(e, hipEventElapsedTime(ms, e->ev0, e->ev1));
+    return SW_OK;
+}
+
+SW_API int sw_engine_trim(sw_engine *e) {
+    if (!e) return SW_E_INVALID;
+    SW_HIP(e, hipSetDevice(e->device));
+    e->pool->release(false);
     return SW_OK;
 }
 

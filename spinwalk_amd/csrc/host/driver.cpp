@@ -42,7 +42,16 @@ int fail(int code, const std::string &m) {
 struct DevBuf {
     void *p = nullptr;
     ~DevBuf() { if (p) (void)hipFree(p); }
-    hipError_t alloc(size_t n) { return n ? hipMalloc(&p, n) : hipSuccess; }
+    // once more without the memory of dropped phantoms that the engine keeps
+    hipError_t alloc(sw_engine *eng, size_t n) {
+        if (!n) return hipSuccess;
+        hipError_t e = hipMalloc(&p, n);
+        if (e == hipErrorOutOfMemory && sw_engine_trim(eng) == SW_OK) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, n);
+        }
+        return e;
+    }
 };
 
 // Host copy of a trajectory chunk (hundreds of MB) split over host threads: one
@@ -170,10 +179,11 @@ int run_phantom(sw_engine *eng, swhost::Config &c, size_t iph, std::vector<float
     (void)hipMemGetInfo(&fr, &tot);
     const size_t need = 24 * (size_t)n + 4 * m1_slice * n_sc + t_slice * n_sc +
                         (streamed ? 2 * 4 * xc : 4 * x_slice * n_sc);
+    if (need > fr && sw_engine_trim(eng) == SW_OK) (void)hipMemGetInfo(&fr, &tot);
     if (need > fr) return fail(SW_E_NOMEM, "not enough device memory for the spin buffers");
-    const bool x_failed = streamed ? (dXa.alloc(4 * xc) != hipSuccess || dXb.alloc(4 * xc) != hipSuccess)
-                                   : dX1.alloc(XYZ1.size() * 4) != hipSuccess;
-    if (dM0.alloc(M0.size() * 4) || dX0.alloc(XYZ0.size() * 4) || dM1.alloc(M1.size() * 4) || dT.alloc(T.size()) ||
+    const bool x_failed = streamed ? (dXa.alloc(eng, 4 * xc) != hipSuccess || dXb.alloc(eng, 4 * xc) != hipSuccess)
+                                   : dX1.alloc(eng, XYZ1.size() * 4) != hipSuccess;
+    if (dM0.alloc(eng, M0.size() * 4) || dX0.alloc(eng, XYZ0.size() * 4) || dM1.alloc(eng, M1.size() * 4) || dT.alloc(eng, T.size()) ||
         x_failed)
         return fail(SW_E_HIP, "hipMalloc failed");
     // the device outputs start from the host buffers (the reference's d_M1 = M1)
@@ -202,7 +212,7 @@ int run_phantom(sw_engine *eng, swhost::Config &c, size_t iph, std::vector<float
         ru_stride = 3 * steps + 64;
         std::vector<float> rn(rn_stride * n), ru(ru_stride * n);
         sw_replay_fill(c.p.seed, 0, n, rn.data(), rn_stride, ru.data(), ru_stride, 16);
-        if (dRN.alloc(rn.size() * 4) || dRU.alloc(ru.size() * 4) ||
+        if (dRN.alloc(eng, rn.size() * 4) || dRU.alloc(eng, ru.size() * 4) ||
             hipMemcpy(dRN.p, rn.data(), rn.size() * 4, hipMemcpyHostToDevice) ||
             hipMemcpy(dRU.p, ru.data(), ru.size() * 4, hipMemcpyHostToDevice))
             return fail(SW_E_HIP, "replay upload failed");

@@ -111,7 +111,7 @@ class SwWalkStats(C.Structure):
 
 # Every entry point include/spinwalk_engine.h declares (checked by the ABI test).
 EXPORTS = (
-    "sw_engine_create", "sw_engine_destroy", "sw_last_error", "sw_device_info", "sw_device_count",
+    "sw_engine_create", "sw_engine_destroy", "sw_engine_trim", "sw_last_error", "sw_device_info", "sw_device_count",
     "sw_version", "sw_params_prepare", "sw_timing_scale", "sw_tesla2deg", "sw_init_positions",
     "sw_replay_fill", "sw_phantom_create", "sw_phantom_create_device", "sw_phantom_destroy",
     "sw_phantom_info", "sw_phantom_download", "sw_phantom_generate", "sw_sequence_create", "sw_sequence_destroy", "sw_walk_device", "sw_walk_device_noalloc", "sw_walk_host",
@@ -179,6 +179,7 @@ def load():
     L.sw_probe_gather_device.argtypes = [_P, _P, C.c_uint64, C.c_uint32, C.c_uint32, C.c_uint64, _P, _P,
                                          C.POINTER(C.c_float)]
     L.sw_stream_sync.argtypes = [_P, _P]
+    L.sw_engine_trim.argtypes = [_P]
     L.sw_batch_create.argtypes = [_P, C.POINTER(SwBatchItem), C.c_uint32, C.POINTER(_P)]
     L.sw_batch_run.argtypes = [_P, _P, C.POINTER(SwWalkStats), C.POINTER(SwWalkStats)]
     L.sw_batch_destroy.argtypes = [_P]
@@ -414,6 +415,10 @@ class Engine:
     def _check(self, rc, what):
         if rc != SW_OK:
             raise EngineError(f"{what}: {self.L.sw_last_error(self.h).decode()} ({rc})")
+
+    def trim(self):
+        """Gives back the device memory of dropped phantoms that the engine keeps for the next ones."""
+        self._check(self.L.sw_engine_trim(self.h), "sw_engine_trim")
 
     def last_error(self):
         return self.L.sw_last_error(self.h).decode()
