@@ -628,9 +628,16 @@ SW_API void sw_phantom_destroy(sw_phantom *ph) {
     if (!ph) return;
     (void)hipSetDevice(ph->device);
     if (ph->arena) {
-        // walks of any stream may still gather from it, as hipFree would wait for them
-        if (hipDeviceSynchronize() == hipSuccess) ph->pool->put(ph->arena, ph->arena_bytes);
-        else dev_free(ph->arena);
+        // Walks of any stream may still gather from it.  hipFree waits for the device before
+        // it frees, 2 us when idle, and may be called beside a relaxed capture, which
+        // hipDeviceSynchronize would invalidate.
+        void *mark = nullptr;
+        if (hipMalloc(&mark, 1) == hipSuccess && hipFree(mark) == hipSuccess) {
+            ph->pool->put(ph->arena, ph->arena_bytes);
+        } else {
+            (void)hipGetLastError();
+            dev_free(ph->arena);
+        }
     }
     delete ph;
 }
