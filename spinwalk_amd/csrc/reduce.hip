@@ -65,14 +65,16 @@ __device__ __forceinline__ void reduce_block(const ReduceItem &r, uint32_t b) {
     for (uint32_t j = 0; j < r.pieces; j++) {
         const uint64_t s0 = first + (uint64_t)j * kPiece;
         if (s0 >= r.n) break;
+        const uint32_t left = (uint32_t)(r.n - s0);
+        const uint64_t base = s0 * r.n_te + te;
         R mx[kPerThread], my[kPerThread];
         uint32_t lab[kPerThread];
         #pragma unroll
         for (uint32_t k = 0; k < kPerThread; k++) {
-            const uint64_t s = s0 + k * kThreads + threadIdx.x;
-            const uint64_t o = s * r.n_te + te;
+            const uint32_t i = k * kThreads + threadIdx.x;
+            const uint64_t o = base + (uint64_t)i * r.n_te;
             lab[k] = ~0u;
-            if (s < r.n) {
+            if (i < left) {
                 lab[k] = r.T[o];
                 if (ALL) { mx[k] = M1[3 * o]; my[k] = M1[3 * o + 1]; }
             }
@@ -80,15 +82,17 @@ __device__ __forceinline__ void reduce_block(const ReduceItem &r, uint32_t b) {
         if (!ALL) {
             #pragma unroll
             for (uint32_t k = 0; k < kPerThread; k++) {
-                const uint64_t o = (s0 + k * kThreads + threadIdx.x) * r.n_te + te;
+                const uint64_t o = base + (uint64_t)(k * kThreads + threadIdx.x) * r.n_te;
                 if (lab[k] - lab0 < kLabels) { mx[k] = M1[3 * o]; my[k] = M1[3 * o + 1]; }
             }
         }
         #pragma unroll
-        for (uint32_t l = 0; l < kLabels; l++)
+        for (uint32_t l = 0; l < kLabels; l++) {
+            if (lab0 + l >= r.n_sub) break;
             #pragma unroll
             for (uint32_t k = 0; k < kPerThread; k++)
                 if (lab[k] == lab0 + l) { v[l][0] += (double)mx[k]; v[l][1] += (double)my[k]; v[l][2] += 1.0; }
+        }
     }
     #pragma unroll
     for (uint32_t l = 0; l < kLabels; l++) {
@@ -119,7 +123,8 @@ __device__ __forceinline__ void finish_pair(const ReduceItem &r, uint32_t pair) 
     if (threadIdx.x == 0) { out[0] = v[0]; out[1] = v[1]; out[2] = v[2]; }
 }
 
-__global__ __launch_bounds__(kThreads) void reduce_pass1(const ReduceItem r) { reduce_block(r, blockIdx.x); }
+template <class R, bool ALL>
+__global__ __launch_bounds__(kThreads) void reduce_pass1(const ReduceItem r) { reduce_block<R, ALL>(r, blockIdx.x); }
 __global__ __launch_bounds__(kThreads) void reduce_pass2(const ReduceItem r) { finish_pair(r, blockIdx.x); }
 
 // items[] in device memory: the last item whose first block (pair) is at or before
@@ -162,7 +167,10 @@ bool reduce_plan(ReduceItem &r) {
 uint64_t reduce_partial_len(const ReduceItem &r) { return 3ull * r.n_chunks * r.pairs; }
 
 hipError_t launch_echo_reduce(const ReduceItem &r, hipStream_t s) {
-    if (r.blocks) hipLaunchKernelGGL(reduce_pass1, dim3(r.blocks), dim3(kThreads), 0, s, r);
+    const bool all = r.n_sub <= kLabels;
+    const auto pass1 = r.f64 ? (all ? reduce_pass1<double, true> : reduce_pass1<double, false>)
+                             : (all ? reduce_pass1<float, true> : reduce_pass1<float, false>);
+    if (r.blocks) hipLaunchKernelGGL(pass1, dim3(r.blocks), dim3(kThreads), 0, s, r);
     if (r.pairs) hipLaunchKernelGGL(reduce_pass2, dim3(r.pairs), dim3(kThreads), 0, s, r);
     return hipGetLastError();
 }
