@@ -1052,8 +1052,11 @@ double voxel_step(const sw_sequence &q, const sw::WalkArgs &a, bool smallest) {
     return q.step_max * s2g;
 }
 
+// Recorded trajectories wait for their stores, not for lines: the line of short steps
+// (1e5 spins of 200 steps of 1.26 voxels on 400^3 792 us unsorted, 843 sorted).
 bool order_pays(const sw_sequence &q, const sw::WalkArgs &a, int field, bool replay) {
-    return sw::order_pays(a.n_local, sw::walk_mode(a, field, replay ? 1 : 0).bytes, voxel_step(q, a, true));
+    return sw::order_pays(a.n_local, sw::walk_mode(a, field, replay ? 1 : 0).bytes,
+                          a.record_traj ? 0. : voxel_step(q, a, true));
 }
 
 bool cap_pays(sw::CapKind kind, const sw_sequence &q, const sw::WalkArgs &a, int field, uint64_t n_all) {
