@@ -224,8 +224,8 @@ SW_HD_INLINE bool stage_wanted(const WalkArgs &a, bool replay) {
 }
 
 // The kernel a walk takes.  Production walks of a scan with one TR, and those that
-// record trajectories, take the step loop of walk_prod.hpp; scans with dummy TRs
-// keep the general loop, whose TR set-up is the cheaper one (the 1000^3 bSSFP
+// record trajectories (single walks of few rows apart: launch_fp), take the step loop of
+// walk_prod.hpp; scans with dummy TRs keep the general loop, whose TR set-up is the cheaper one (the 1000^3 bSSFP
 // batch of 100 dummy TRs: 117.2 ms against 121.6 ms; the FoV sweep, one TR each:
 // 120.4 against 118.7 ms).  The general loop is compiled per boundary rule.
 enum Variant : int { VARIANT_PLAIN = 0, VARIANT_CROSS = 1, VARIANT_ONE_TR = 2, VARIANT_TRAJ = 3, VARIANTS = 4 };

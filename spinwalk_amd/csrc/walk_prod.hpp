@@ -239,6 +239,8 @@ __device__ __forceinline__ bool prod_outside(ArgsPtr a, const Hot &h, const floa
     return ok;
 }
 
+enum : int { TRAJ_NONE = 0, TRAJ_DIRECT = 1, TRAJ_STAGED = 2 };
+
 // Recorded positions on their way to XYZ1.  Each spin has a row of its own, so a
 // store per step is 64 pieces of 12 bytes in 64 lines, and the L2 sends nearly each of
 // them on by itself: 63 M write requests, 3.3 GB, for the 0.96 GB of 1e5 spins and 800
@@ -252,37 +254,27 @@ __device__ __forceinline__ bool prod_outside(ArgsPtr a, const Hot &h, const floa
 // 8e4 1.21 and 0.82).  Compiled for 4 waves a SIMD, which is what the rings leave room for
 // and where nothing of the step loop spills.
 // A lane's words: absolute word w (row words from the row's 64-byte boundary) in
-// piece w / 4 mod 8, the pieces 64 lanes apart.  Without room in LDS
-// (WalkArgs::stage) every step is written as it comes.
+// piece w / 4 mod 8, the pieces 64 lanes apart.
 typedef uint32_t Piece __attribute__((ext_vector_type(4)));
 typedef uint32_t PieceOut __attribute__((ext_vector_type(4), aligned(4)));
 template <bool IDX32> struct Recorder {
-    bool on;                     // staged
     uint32_t ring;               // this lane's place in the wave's ring, axis_tab[ring ..]
     uint32_t first, w, done;     // words: the row's first, the next, the first not yet written
     float vs[3];
     __device__ Recorder(ArgsPtr a, ViewPtr, uint64_t xoff)
-        : on(a->stage), ring(stage_ring<IDX32>(*a) + 4 * (threadIdx.x & 63)), vs{a->vsf[0], a->vsf[1], a->vsf[2]} {
-        first = w = done = (uint32_t)((uintptr_t)(a->XYZ1 + xoff) / 4) & (on ? 15u : 0u);
+        : ring(stage_ring<IDX32>(*a) + 4 * (threadIdx.x & 63)), vs{a->vsf[0], a->vsf[1], a->vsf[2]} {
+        first = w = done = (uint32_t)((uintptr_t)(a->XYZ1 + xoff) / 4) & 15u;
     }
     __device__ bool any() const { return w != first; }
     // word i's place
     __device__ uint32_t place(uint32_t i) const { return ring + (i & 28u) * 64 + (i & 3u); }
     template <int NV> __device__ void add(ArgsPtr a, ViewPtr xv, uint64_t xoff, const float y[3]) {
-        if (!on) {
-            #pragma unroll
-            for (int v = 0; v < NV; v++) {
-                float *dst = SW_VIEW(a, xv, v, XYZ1) + xoff + w;
-                for (int i = 0; i < 3; i++) dst[i] = y[i] * vs[i];
-            }
-        } else {
-            for (uint32_t i = 0; i < 3; i++) axis_tab[place(w + i)] = __float_as_uint(y[i] * vs[i]);
-        }
+        for (uint32_t i = 0; i < 3; i++) axis_tab[place(w + i)] = __float_as_uint(y[i] * vs[i]);
         w += 3;
     }
     // Called by every lane of the wave that still walks.
     template <int NV> __device__ void spill(ArgsPtr a, ViewPtr xv, uint64_t xoff) {
-        if (on && __builtin_amdgcn_ballot_w64(w - (done & ~15u) > 29) != 0) write<NV>(a, xv, xoff);
+        if (__builtin_amdgcn_ballot_w64(w - (done & ~15u) > 29) != 0) write<NV>(a, xv, xoff);
     }
     template <int NV> __device__ void write(ArgsPtr a, ViewPtr xv, uint64_t xoff) {
         // a row's first words, up to its first 64-byte boundary
@@ -320,6 +312,7 @@ template <bool IDX32> struct Recorder {
             for (int v = 0; v < NV; v++) *(PieceOut *)(SW_VIEW(a, xv, v, XYZ1) + o + j4) = p;
         }
     }
+    template <int NV> __device__ void finish(ArgsPtr a, ViewPtr xv, uint64_t xoff) { words<NV>(a, xv, xoff, w); }
     // this lane's words up to `end`, one by one
     template <int NV> __device__ void words(ArgsPtr a, ViewPtr xv, uint64_t xoff, uint32_t end) {
         for (; done < end; done++) {
@@ -330,10 +323,31 @@ template <bool IDX32> struct Recorder {
     }
 };
 
+// Recorded positions written as they come: few rows, or no room in LDS (WalkArgs::stage).
+// A walk of its own instead of a branch per step: 2e4 spins 217 -> 210 us.
+struct DirectRecorder {
+    uint64_t at;                 // the next word of XYZ1
+    float vs[3];
+    bool some = false;
+    __device__ DirectRecorder(ArgsPtr a, ViewPtr, uint64_t xoff) : at(xoff), vs{a->vsf[0], a->vsf[1], a->vsf[2]} {}
+    __device__ bool any() const { return some; }
+    template <int NV> __device__ void add(ArgsPtr a, ViewPtr xv, uint64_t, const float y[3]) {
+        #pragma unroll
+        for (int v = 0; v < NV; v++) {
+            float *dst = SW_VIEW(a, xv, v, XYZ1) + at;
+            for (int i = 0; i < 3; i++) dst[i] = y[i] * vs[i];
+        }
+        at += 3;
+        some = true;
+    }
+    template <int NV> __device__ void spill(ArgsPtr, ViewPtr, uint64_t) {}
+    template <int NV> __device__ void finish(ArgsPtr, ViewPtr, uint64_t) {}
+};
+
 // One spin.  ONE_TR: the scan has no dummy TRs, so every lane of the wave that
 // still walks is at the same attempt, and the attempt counter and the draw's
 // first products run on the scalar unit.
-template <class Rec, class Phase, bool IDX32, int NV, bool ONE_TR, bool TRAJ>
+template <class Rec, class Phase, bool IDX32, int NV, bool ONE_TR, int TRAJ>
 __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li, uint64_t &n_acc, uint32_t &n_rej) {
     using R = typename Phase::R;
     using RI = RecIdx<IDX32>;
@@ -367,7 +381,7 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
         typename Rec::T raw = rec_load<Rec, IDX32>(a->rec, vx.rec);
         uint32_t ts = Rec::label(raw);                                 // :103
         float step[3];
-        [[maybe_unused]] Recorder<IDX32> rec1(a, xv, xoff);
+        [[maybe_unused]] typename std::conditional<TRAJ == TRAJ_STAGED, Recorder<IDX32>, DirectRecorder>::type rec1(a, xv, xoff);
         uint64_t att = 0;
         uint32_t itr = 0, last_rej = 0;
         ProdDraw q = prod_draw<ONE_TR>(0, m_hi, m_lo, k0, k1);
@@ -469,7 +483,7 @@ __device__ __forceinline__ int walk_spin_prod(ArgsPtr a, ViewPtr xv, uint32_t li
             if (last) { ++d; tp = 0; break; }                          // every TR done
         }
         if constexpr (TRAJ) {
-            if (rec1.on) rec1.template words<NV>(a, xv, xoff, rec1.w);   // the row's last words, also of a lost spin
+            rec1.template finish<NV>(a, xv, xoff);                     // the row's last words, also of a lost spin
             recorded = rec1.any();
         }
     }
@@ -503,8 +517,13 @@ __device__ __forceinline__ void prod_block(ArgsPtr a, ViewPtr xv, uint32_t n_vie
     uint32_t n_rej = 0, lost = 0;
     for (uint32_t k = 0; k < spl; k++) {
         const uint32_t t = t0 + k * blockDim.x;
-        if (t < a->n_local)
-            lost += walk_spin_prod<Rec, Phase, IDX32, NV, ONE_TR, TRAJ>(a, xv, a->order ? a->order[t] : t, n_acc, n_rej) == ST_LOST;
+        if (t >= a->n_local) continue;
+        const uint32_t li = a->order ? a->order[t] : t;
+        int st;
+        if constexpr (!TRAJ) st = walk_spin_prod<Rec, Phase, IDX32, NV, ONE_TR, TRAJ_NONE>(a, xv, li, n_acc, n_rej);
+        else if (a->stage) st = walk_spin_prod<Rec, Phase, IDX32, NV, ONE_TR, TRAJ_STAGED>(a, xv, li, n_acc, n_rej);
+        else st = walk_spin_prod<Rec, Phase, IDX32, NV, ONE_TR, TRAJ_DIRECT>(a, xv, li, n_acc, n_rej);
+        lost += st == ST_LOST;
     }
     const uint64_t s_acc = wave_sum_u64(n_acc), s_rej = wave_sum_u64(n_rej), s_lost = wave_sum_u64(lost);
     if ((threadIdx.x & 63) == 0) {
