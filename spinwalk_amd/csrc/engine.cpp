@@ -1070,6 +1070,11 @@ bool cap_pays(sw::CapKind kind, const sw_sequence &q, const sw::WalkArgs &a, int
 
 constexpr uint32_t kBatchWaves = 5;
 
+uint32_t single_general(const sw_sequence &q, const sw::WalkArgs &a, int precision) {
+    return sw::general_loop(a.n_local, precision == SW_PREC_F64, voxel_step(q, a, true),
+                            !a.closed && a.n_sub > sw::kTissueLdsMax);
+}
+
 // Trajectories and replayed draws stream from HBM and keep every wave they can.
 uint32_t single_cap(const sw_sequence &q, const sw::WalkArgs &a, int field, bool replay) {
     return !replay && !a.record_traj && cap_pays(a.pairs ? sw::CAP_PAIRS : sw::CAP_SINGLE, q, a, field, a.n_local);
@@ -1100,6 +1105,7 @@ SW_API int sw_walk_device(sw_engine *e, const sw_phantom *ph, const sw_sequence 
         if (rc) return rc;
         a.order = e->d_order;
     }
+    a.general = single_general(*q, a, o->precision);
     a.cap = single_cap(*q, a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(e->d_counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));
@@ -1164,6 +1170,7 @@ SW_API int sw_walk_device_noalloc(sw_engine *e, const sw_phantom *ph, const sw_s
             a.order = order;
         }
     }
+    a.general = single_general(*q, a, o->precision);
     a.cap = single_cap(*q, a, field, o->rng == SW_RNG_REPLAY);
     SW_HIP(e, sw::launch_zero_u64(a.counters, 4, s));
     if (stats) SW_HIP(e, hipEventRecord(e->ev0, s));

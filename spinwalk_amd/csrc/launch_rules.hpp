@@ -1,6 +1,6 @@
 // launch_rules.hpp -- how a walk is launched, as rules on its sizes: whether its spins
-// are visited sorted, how many a wave carries, and whether the waves on a SIMD are
-// capped.  None changes a result.  Plain C++.
+// are visited sorted, how many a wave carries, which loop walks them, and whether the
+// waves on a SIMD are capped.  None changes a result.  Plain C++.
 #pragma once
 #include <math.h>
 #include <stdint.h>
@@ -49,6 +49,21 @@ inline uint32_t unsorted_spins(double step) {
 }
 inline bool order_pays(uint32_t n_local, uint64_t rec_bytes, double step) {
     return n_local > unsorted_spins(step) && rec_bytes >= kUnsortedBytes;
+}
+
+// Whether a single walk of one TR in single precision takes the general loop and not that
+// of walk_prod.hpp, whose rare blocks (walls, crossings) are the longer ones where a wave
+// has a SIMD to itself.  That shows between the half-filled waves and two waves a SIMD
+// where a wave meets such a block at nearly every step: long steps, or crossings that read
+// their probability from global memory (more tissues than the LDS tables take).  General
+// loop over production loop, 400 steps:
+//                                      1e3 spins  3e4    3.3e4  6.5e4  1e5    1.4e5  4e5
+//   2 tissues, 128^3, step 0.2          1.09      1.05   1.00   0.99   1.01   1.04   1.04
+//                          0.63         1.02      0.99   0.95   0.95   0.96   0.97   1.01
+//   20 tissues, permeable, step 0.32    1.1 (2e3)        0.92   0.92   0.94   0.96   1.0 (5e5)
+// In double precision the production loop is the faster by 1.04 to 1.14 throughout.
+inline bool general_loop(uint32_t n_local, bool f64, double step, bool global_crossings) {
+    return !f64 && n_local > 32u * 1024 && n_local <= 128u * 1024 && (step >= 0.5 || global_crossings);
 }
 
 // Whether the waves on a SIMD are held to kCapWaves (4) in a single walk, or a batch's to

@@ -169,6 +169,7 @@ struct WalkArgs {
     uint32_t        pairs;        // 1: a single production walk takes two attempts per trip of its step loop
     uint32_t        closed;       // 1: no crossing probability between two tissues is above 0
     uint32_t        super_blocks; // 1: the packed records are grouped in super-blocks (kSuper)
+    uint32_t        general;      // 1: a single walk of one TR takes the general loop (general_loop)
     uint32_t        cap;          // 1: a single walk holds the waves on a SIMD to kCapWaves (capped_lds)
     const RfPulse  *rf;           // [n_rf]; entry 0 unused (excitation)
     uint32_t        n_rf;

@@ -1706,7 +1706,9 @@ hipError_t launch_fp(const WalkArgs &a, hipStream_t s, dim3 grid, dim3 block) {
             // 4e4 spins 219 us against 238, 7e4 280 against 303; in double 371 against 316).
             if (!a.stage && sizeof(typename P::R) == 4) return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
             return launch_prod<F, P, false, true>(a, s, grid, block);
-        case VARIANT_ONE_TR: return launch_prod<F, P, true, false>(a, s, grid, block);
+        case VARIANT_ONE_TR:
+            if (a.general) return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
+            return launch_prod<F, P, true, false>(a, s, grid, block);
         default: return launch_fp_loop<Rng, F, P, false>(a, s, grid, block);
         }
     }

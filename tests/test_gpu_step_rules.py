@@ -22,6 +22,22 @@ def test_sorted_equals_unsorted(engine, n):
         assert a["stats"][k] == b["stats"][k]
 
 
+@pytest.mark.parametrize("n", [32769, 40001])
+@pytest.mark.parametrize("n_sub,fov", [(2, 27.1), (2, 60.0), (20, 100.0)])     # steps of 0.74, 0.34 and 0.2 voxels
+def test_general_loop_equals_production_loop(engine, n, n_sub, fov):
+    """The whole walk takes the general loop (or, at 0.34, does not), its parts of up to
+    32768 spins the production loop."""
+    m, f = cases.blocky_phantom((64,) * 3, n_labels=n_sub, seed=3)
+    pxy = np.random.default_rng(2).uniform(0.2, 0.8, (n_sub, n_sub)).tolist()
+    case = cases.make_case(cases.gre(n_sub, TE=900, dt=50, P_XY=pxy), m, f, fov, n_spins=n)
+    whole = run(engine, case)
+    parts = [run(engine, case, spin_offset=o, n=min(20000, n - o)) for o in range(0, n, 20000)]
+    for k in ("M1", "T", "XYZ1"):
+        np.testing.assert_array_equal(whole[k], np.concatenate([p[k] for p in parts]))
+    for k in ("n_lost", "n_steps", "n_attempts"):
+        assert whole["stats"][k] == sum(p["stats"][k] for p in parts)
+
+
 @pytest.mark.parametrize("dummies,waves", [(0, 4), (4, 5)])
 def test_default_waves_of_a_batch(engine, dummies, waves):
     import torch

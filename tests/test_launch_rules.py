@@ -14,6 +14,7 @@ CODE = r'''
 #include "%s"
 extern "C" unsigned unsorted(double step) { return sw::unsorted_spins(step); }
 extern "C" int order(unsigned n, unsigned long long bytes, double step) { return sw::order_pays(n, bytes, step); }
+extern "C" int general(unsigned n, int f64, double step, int global) { return sw::general_loop(n, f64 != 0, step, global != 0); }
 extern "C" double reach(double bytes, double vox, double n, int sorted, double step, double steps) {
     return sw::cap_reach((unsigned long long)bytes, vox, (unsigned long long)n, sorted != 0, step, steps);
 }
@@ -38,6 +39,7 @@ def rules():
         d_, i = ctypes.c_double, ctypes.c_int
         lib.unsorted.argtypes, lib.unsorted.restype = [d_], ctypes.c_uint
         lib.order.argtypes = [ctypes.c_uint, ctypes.c_ulonglong, d_]
+        lib.general.argtypes = [ctypes.c_uint, i, d_, i]
         lib.reach.argtypes, lib.reach.restype = [d_, d_, d_, i, d_, d_], d_
         lib.window.argtypes, lib.window.restype = [d_, d_, d_, i, d_], d_
         lib.cap.argtypes = [i, i, d_, d_, d_]
@@ -54,6 +56,12 @@ def test_sorting_begins_at_fewer_spins_where_steps_are_long(rules):
     for step in (float("inf"), float("nan")):
         assert 90000 <= rules.unsorted(step) <= 212992
     assert all(rules.unsorted(s / 100) >= rules.unsorted((s + 1) / 100) for s in range(1000))
+
+
+def test_general_loop_between_half_waves_and_two_waves(rules):
+    for n, on in ((32768, False), (32769, True), (131072, True), (131073, False)):
+        assert bool(rules.general(n, 0, 0.5, 0)) == on and bool(rules.general(n, 0, 0.1, 1)) == on
+        assert not rules.general(n, 1, 0.5, 1) and not rules.general(n, 0, 0.49, 0)
 
 
 def _reach(rules, side, bytes_per_voxel, n, step, steps, is_sorted=1):
