@@ -169,14 +169,13 @@ struct WalkArgs {
     uint32_t        pairs;        // 1: a single production walk takes two attempts per trip of its step loop
     uint32_t        closed;       // 1: no crossing probability between two tissues is above 0
     uint32_t        super_blocks; // 1: the packed records are grouped in super-blocks (kSuper)
-    uint32_t        general;      // 1: a single walk of one TR takes the general loop (general_loop)
     uint32_t        cap;          // 1: a single walk holds the waves on a SIMD to kCapWaves (capped_lds)
     const RfPulse  *rf;           // [n_rf]; entry 0 unused (excitation)
     uint32_t        n_rf;
     const int32_t  *TE_t;         uint32_t n_te;
     const int32_t  *deph_t;       const float *deph_deg; uint32_t n_deph;
     const int32_t  *grad_t;       const float *gx, *gy, *gz; uint32_t n_grad;
-    uint32_t        stage;        // 1: the workgroup has kStageBytes of LDS a lane after its tables (stage_column)
+    uint32_t        stage;        // 1: the workgroup has kStageBytes of LDS a lane after its tables (stage_ring)
     const Excitation *exc;        // [n_dummy + 1]
     float           exc_s, exc_c; // param.s, param.c
     double          exc_sd, exc_cd;
@@ -204,6 +203,8 @@ struct WalkArgs {
 
     // ---- counters: [0] lost, [1] replay exhausted, [2] accepted steps, [3] attempts
     unsigned long long *counters;
+
+    uint32_t        general;      // 1: a single walk of one TR takes the general loop (general_loop)
 };
 
 // Production walks in the 32-bit mode with at most kTissueLdsMax tissues keep

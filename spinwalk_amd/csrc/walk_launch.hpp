@@ -14,14 +14,14 @@ namespace sw {
 // prec: 0 f32, 1 f32+Kahan, 2 f64.
 hipError_t launch_walk(const WalkArgs &a, int rng, int field, int prec, hipStream_t s);
 
-// The index mode the walk takes for a phantom and field format: 32-bit record
-// offsets with per-axis LDS tables of `lds` bytes, or 64-bit arithmetic.
 // The cap on the waves of a SIMD: a CU's LDS holds 4 workgroups of 256 spins (4
 // waves, one a SIMD) of this much, and not 5.
 constexpr uint32_t kCapWaves = 4;
 constexpr size_t kLdsPerCu = 160 * 1024, kCapLds = (2 * kLdsPerCu / (2 * kCapWaves + 1)) & ~(size_t)1023;
 inline size_t capped_lds(const WalkArgs &a, size_t lds) { return a.cap && lds < kCapLds ? kCapLds : lds; }
 
+// The index mode the walk takes for a phantom and field format: 32-bit record
+// offsets with per-axis LDS tables of `lds` bytes, or 64-bit arithmetic.
 struct WalkMode { bool idx32; size_t lds; uint64_t bytes; };   // bytes: the gathered records
 WalkMode walk_mode(const WalkArgs &a, int field, int rng);
 
