@@ -264,6 +264,9 @@ def main_tiles(args, torch, E, W, eng, stream, dev):
         log(f"[bench]   mixed: tile {w['tile']} {w['seq']} scale {w['scale']:.3g} label {w['label']}: signal "
             f"{w['signal']:.6g} vs FP64 {w['f64']:.6g}, abs {w['abs_err']:.2e}, rel {w['rel_err']:.2e}")
 
+    # scans of one TR walk in the production loop, those with dummy TRs in the general one
+    kernel = "walk_batch_kernel" if any(t["params"].n_dummy_scan for t in tiles) else "walk_batch_prod_kernel"
+
     def roofline(res, field, tag):
         bpe = 5 if field == E.SW_FIELD_F32 else 3           # u8 mask + field bytes per spin-step
         kernel_s = res["stats"]["kernel_ms"] * 1e-3
@@ -285,7 +288,7 @@ def main_tiles(args, torch, E, W, eng, stream, dev):
         return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_note": traffic_note,
                 "traffic_rate": None if traffic is None else traffic / kernel_s / 1e9,
-                "bytes_per_spin_step": bpe, "kernel_ms": res["stats"]["kernel_ms"], "kernel": "walk_batch_kernel"}
+                "bytes_per_spin_step": bpe, "kernel_ms": res["stats"]["kernel_ms"], "kernel": kernel}
 
     mixed_tag = f"{args.precision or 'kahan'}_{args.field or 'q16'}"
     out = {
