@@ -10,7 +10,8 @@
 // against the general loop (walk_spin) this one
 // - counts attempts on the scalar unit where they are uniform, with the two draw
 //   products that then are uniform too, and keeps the round keys in scalar
-//   registers (67 instead of 96 instructions a draw);
+//   registers (with the rest, 87.5 instead of 94.4 VALU instructions a wave-step on the
+//   FoV sweep's FP32 batch);
 // - holds the gathered record in place: a lane that stays in its voxel keeps the
 //   one it has, so neither record index nor field is selected per step;
 // - reads T1 and T2 at events instead of at every change of tissue;
@@ -19,7 +20,9 @@
 //   loop's scalar registers hold no more than it uses.
 // Measured, start of this change against now: 200 k spins, 1201 time points,
 // permeable, FP64: 2.39 -> 1.91 ms; 12 phantoms, GRE/SE/PGSE, Kahan + int16 batch:
-// 7.53 -> 7.21 ms; 64 tiles of the FoV sweep, FP32 batch: 120.4 -> 118.5 ms.
+// 7.53 -> 7.21 ms; 64 tiles of the FoV sweep, FP32 batch: 120.4 -> 118.5 ms.  Where walls
+// are met at nearly every step and a wave has a SIMD to itself, its longer rare blocks
+// cost more than that (general_loop).
 #pragma once
 
 namespace sw {
